@@ -60,14 +60,48 @@ __device__ __forceinline__ constexpr float c20(int j) {
 }
 __device__ __forceinline__ constexpr float s20(int j) { return c20(j - 5); }
 
-// W_N^m with sign S: exp(S * 2 pi i m / N), for N dividing 48 or 20
+// cos(2 pi j / 64) for the radices 32 and 64
+__device__ __forceinline__ constexpr float c64q(int q) {  // q in [0, 16]
+  return q == 0 ? 1.0f : q == 1 ? 0.99518472667219693f : q == 2 ? 0.98078528040323044f
+       : q == 3 ? 0.95694033573220886f : q == 4 ? 0.92387953251128674f : q == 5 ? 0.88192126434835503f
+       : q == 6 ? 0.83146961230254524f : q == 7 ? 0.77301045336273696f : q == 8 ? 0.70710678118654752f
+       : q == 9 ? 0.63439328416364549f : q == 10 ? 0.55557023301960222f : q == 11 ? 0.47139673682599764f
+       : q == 12 ? 0.38268343236508977f : q == 13 ? 0.29028467725446236f : q == 14 ? 0.19509032201612827f
+       : q == 15 ? 0.09801714032956060f : 0.0f;
+}
+__device__ __forceinline__ constexpr float c64(int j) {
+  const int m = ((j % 64) + 64) % 64;
+  const int q = (m <= 32) ? m : 64 - m;
+  return (q <= 16) ? c64q(q) : -c64q(32 - q);
+}
+__device__ __forceinline__ constexpr float s64(int j) { return c64(j - 16); }
+
+// cos(2 pi j / 40) for the radix 40
+__device__ __forceinline__ constexpr float c40q(int q) {  // q in [0, 10]
+  return q == 0 ? 1.0f : q == 1 ? 0.98768834059513773f : q == 2 ? 0.95105651629515357f
+       : q == 3 ? 0.89100652418836786f : q == 4 ? 0.80901699437494742f : q == 5 ? 0.70710678118654752f
+       : q == 6 ? 0.58778525229247313f : q == 7 ? 0.45399049973954675f : q == 8 ? 0.30901699437494742f
+       : q == 9 ? 0.15643446504023087f : 0.0f;
+}
+__device__ __forceinline__ constexpr float c40(int j) {
+  const int m = ((j % 40) + 40) % 40;
+  const int q = (m <= 20) ? m : 40 - m;
+  return (q <= 10) ? c40q(q) : -c40q(20 - q);
+}
+__device__ __forceinline__ constexpr float s40(int j) { return c40(j - 10); }
+
+// W_N^m with sign S: exp(S * 2 pi i m / N), for N dividing 48, 20, 64 or 40
 template <int N, int S>
 __device__ __forceinline__ constexpr float2 wn(int m) {
-  static_assert(48 % N == 0 || 20 % N == 0, "no twiddle constants for this radix");
+  static_assert(48 % N == 0 || 20 % N == 0 || 64 % N == 0 || 40 % N == 0, "no twiddle constants for this radix");
   if constexpr (48 % N == 0)
     return make_float2(c48(m * (48 / N)), (S < 0 ? -1.0f : 1.0f) * s48(m * (48 / N)));
-  else
+  else if constexpr (20 % N == 0)
     return make_float2(c20(m * (20 / N)), (S < 0 ? -1.0f : 1.0f) * s20(m * (20 / N)));
+  else if constexpr (64 % N == 0)
+    return make_float2(c64(m * (64 / N)), (S < 0 ? -1.0f : 1.0f) * s64(m * (64 / N)));
+  else
+    return make_float2(c40(m * (40 / N)), (S < 0 ? -1.0f : 1.0f) * s40(m * (40 / N)));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -150,6 +184,7 @@ __device__ __forceinline__ void dft_split(float2* v) {
 #pragma unroll
   for (int n2 = 0; n2 < R2; n2++) {
     float2 t[R1];
+    if (N >= 40) __builtin_amdgcn_sched_barrier(0);  // one sub-transform's temporaries at a time
 #pragma unroll
     for (int n1 = 0; n1 < R1; n1++) t[n1] = v[R2 * n1 + n2];
     Dft<R1, S>::run(t);
@@ -159,6 +194,7 @@ __device__ __forceinline__ void dft_split(float2* v) {
 #pragma unroll
   for (int k1 = 0; k1 < R1; k1++) {
     float2 t[R2];
+    if (N >= 40) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int n2 = 0; n2 < R2; n2++) t[n2] = a[n2][k1];
     Dft<R2, S>::run(t);
@@ -186,6 +222,22 @@ struct Dft<16, S> {
 template <int S>
 struct Dft<24, S> {
   __device__ __forceinline__ static void run(float2* v) { dft_split<3, 8, S>(v); }
+};
+template <int S>
+struct Dft<32, S> {
+  __device__ __forceinline__ static void run(float2* v) { dft_split<4, 8, S>(v); }
+};
+template <int S>
+struct Dft<40, S> {
+  __device__ __forceinline__ static void run(float2* v) { dft_split<5, 8, S>(v); }
+};
+template <int S>
+struct Dft<48, S> {
+  __device__ __forceinline__ static void run(float2* v) { dft_split<6, 8, S>(v); }
+};
+template <int S>
+struct Dft<64, S> {
+  __device__ __forceinline__ static void run(float2* v) { dft_split<8, 8, S>(v); }
 };
 template <int S>
 struct Dft<10, S> {

@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include "fft2s.h"
+#include "rd_gpu.h"
 
 // minimum waves per SIMD requested from the compiler for the transform kernels (caps VGPRs); the
 // per-kernel values apply to plans of at most 16 values per thread, longer plans use 2
@@ -86,145 +87,6 @@ using namespace dev;
 #ifndef GLIA_NT_ZP
 #define GLIA_NT_ZP 2
 #endif
-
-// ---------------------------------------------------------------------------------------------
-// helpers
-// ---------------------------------------------------------------------------------------------
-// pointers into device global memory (address space 1): loads and stores through them compile to
-// global_* instructions with a uniform base and 32-bit lane offsets instead of flat accesses
-#define GLIA_GLOBAL __attribute__((address_space(1)))
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-// Cache policy of a kernel's global accesses, a template argument of its pointers: bit 0 makes
-// the loads, bit 1 the stores non-temporal (the nt bit: the line streams through the caches instead
-// of being kept for reuse).  Each pass sets its own (GLIA_NT_* below).
-template <int H>
-struct GRefT {
-  GLIA_GLOBAL v2f* p;
-  __device__ __forceinline__ operator float2() const {
-    v2f a;
-    if constexpr ((H & 1) != 0) {
-      a = __builtin_nontemporal_load(p);
-    } else {
-      a = *p;
-    }
-    return make_float2(a.x, a.y);
-  }
-  __device__ __forceinline__ GRefT& operator=(float2 v) {
-    v2f a;
-    a.x = v.x;
-    a.y = v.y;
-    if constexpr ((H & 2) != 0) {
-      __builtin_nontemporal_store(a, p);
-    } else {
-      *p = a;
-    }
-    return *this;
-  }
-};
-template <int H>
-struct GPtrT {
-  GLIA_GLOBAL v2f* p;
-  __device__ __forceinline__ GRefT<H> operator[](unsigned i) const { return GRefT<H>{p + i}; }
-  __device__ __forceinline__ GPtrT operator+(int64_t o) const { return GPtrT{p + o}; }
-  __device__ __forceinline__ explicit operator bool() const { return p != nullptr; }
-};
-using GPtr = GPtrT<0>;
-// 16-byte accesses of the elementwise passes under the same policy bits
-template <int H>
-__device__ __forceinline__ v4f ld4(GLIA_GLOBAL v4f* p) {
-  if constexpr ((H & 1) != 0) {
-    return __builtin_nontemporal_load(p);
-  } else {
-    return *p;
-  }
-}
-template <int H>
-__device__ __forceinline__ void st4(GLIA_GLOBAL v4f* p, v4f v) {
-  if constexpr ((H & 2) != 0) {
-    __builtin_nontemporal_store(v, p);
-  } else {
-    *p = v;
-  }
-}
-template <int H = 0>
-__device__ __forceinline__ GPtrT<H> gptr(const void* q) { return GPtrT<H>{(GLIA_GLOBAL v2f*)q}; }
-
-// complex slot s of a member: work slots below CS_NUM, state-pool entries (history/checkpoints) above
-template <int H = 0>
-__device__ __forceinline__ GPtrT<H> cptr(const MemberDev& M, int s) {
-  return gptr<H>((s < CS_NUM) ? M.c[s] : M.hist[s - CS_NUM]);
-}
-// the same slot as a plain pointer (elementwise kernels)
-__device__ __forceinline__ float2* craw(const MemberDev& M, int s) { return (s < CS_NUM) ? M.c[s] : M.hist[s - CS_NUM]; }
-// a real field viewed as float2 pairs (x[2n], x[2n+1])
-template <int H = 0>
-__device__ __forceinline__ GPtrT<H> rptr2(const MemberDev& M, int r) { return gptr<H>(M.r[r]); }
-
-// wave number with the Nyquist mode zeroed (reference src/cuda/SpectralOperators.cu:63-72)
-__device__ __forceinline__ float wnum(int k, int n) {
-  const int h = n >> 1;
-  return (k < h) ? (float)k : ((k == h) ? 0.f : (float)(k - n));
-}
-
-// spectral preconditioner factor times N^3 (reference src/cuda/DiffCoef.cu:11-63):
-// FFT(B r) = r_hat / (1 + 0.25 dt kbar |w|^2), or r_hat when the denominator is 0
-__device__ __forceinline__ float precf(float pc, float wx, float wy, float wz) {
-  const float v = 1.0f + pc * (wx * wx + wy * wy + wz * wz);
-  return (v == 0.0f) ? 1.0f : 1.0f / v;
-}
-
-// block-wide FP64 reduction of NQ values; thread 0 writes out[0..NQ)
-template <int NQ>
-__device__ __forceinline__ void block_reduce_store(double (&v)[NQ], double* out) {
-  __shared__ double red[NQ][16];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int nw = (blockDim.x + 63) >> 6;
-#pragma unroll
-  for (int q = 0; q < NQ; q++) {
-    double x = v[q];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-    if (lane == 0) red[q][wid] = x;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      double s = 0;
-      for (int w = 0; w < nw; w++) s += red[q][w];
-      out[q] = s;
-    }
-  }
-}
-
-// block-wide sum of one value, result broadcast to every thread
-__device__ __forceinline__ double block_sum_all(double x) {
-  __shared__ double red[16];
-  __shared__ double res;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int nw = (blockDim.x + 63) >> 6;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-  if (lane == 0) red[wid] = x;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double s = 0;
-    for (int w = 0; w < nw; w++) s += red[w];
-    res = s;
-  }
-  __syncthreads();
-  const double r = res;
-  __syncthreads();
-  return r;
-}
-
-// sum of column q of part[nb][nq], identical on every thread (fixed order: deterministic)
-__device__ __forceinline__ double sum_partials(const double* part, int nb, int nq, int q) {
-  double s = 0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) s += part[(int64_t)b * nq + q];
-  return block_sum_all(s);
-}
 
 // ---------------------------------------------------------------------------------------------
 // column kernels (X and Y passes): a tile of 16 adjacent columns (128-byte rows), NT threads per
@@ -524,16 +386,18 @@ k_yf_div(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ t
 }
 
 
-// X pass, forward, closing the divergence: D = i w_x FFT_x(Yx) + FFT_x(Rr) = FFT(div(k grad p)).
+// X pass, forward, closing the divergence: D = i w_x FFT_x(Yx) + FFT_x(Rr) = FFT(div(k grad p)).  With
+// SUM the second input is the sum of slots s_rr and s_rb (the plane pass writes them apart).
 //   XF_MATVEC: w = p - (tau/2) D; partial <p, w>
 //   XF_SETUP : r = tau D (= b - A x for x0 = c); partials ||B b||^2, ||B r||^2, <B r, r>
 //              with b = x + (tau/2) D
 //   XF_D     : out = D
 enum { XF_MATVEC = 0, XF_SETUP = 1, XF_D = 2 };
 
-template <int L, int MODE>
+template <int L, int MODE, bool SUM>
 __global__ void __launch_bounds__(CK<L>::TPB, CK<L>::VPT <= 16 ? GLIA_XF_MINW : 2)
-k_xf_div(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ tw, int s_yx, int s_rr, int s_p, int s_out) {
+k_xf_div(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ tw, int s_yx, int s_rr, int s_rb, int s_p,
+         int s_out) {
   constexpr int H = GLIA_NT_XF;
   const MemberDev& M = mem[blockIdx.y];
   const PcgState* st = M.st;
@@ -555,6 +419,11 @@ k_xf_div(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ t
     const unsigned g = (unsigned)in_row<R1, R2, NT>(t, j) * tl.rs + col;
     a[j] = Yx[g];
     b[j] = Rr[g];
+  }
+  if constexpr (SUM) {
+    GPtrT<H> Rb = cptr<H>(M, s_rb) + tl.base;
+#pragma unroll
+    for (int j = 0; j < K::VIN; j++) b[j] = cadd(b[j], Rb[(unsigned)in_row<R1, R2, NT>(t, j) * tl.rs + col]);
   }
   // the operand of the output stage is loaded before the transforms (a barrier would otherwise
   // keep its loads behind them)
@@ -1479,21 +1348,9 @@ __device__ __forceinline__ void ksp_finish(PcgState* s, int reason, int its) {
   if (reason < s->worst_reason) s->worst_reason = reason;
 }
 
-// start of every CN solve: parameters and a clean iteration state
+// start of a CN solve
 __global__ void k_pcg_begin(const MemberDev* __restrict__ mem, double tau) {
-  if (threadIdx.x != 0) return;
-  PcgState* s = mem[blockIdx.x].st;
-  s->tau = tau;
-  s->beta = s->betaold = s->dpi = s->dpiold = s->alpha = s->bcoef = 0;
-  s->dp = s->rnorm0 = s->ttol = 0;
-  s->i = 0;
-  s->its = 0;
-  s->reason = 0;
-  s->done = 0;
-  if (!s->active) {  // DiffusionSolver::solve returns at once when k_scale == 0
-    s->done = 1;
-    s->solves += 1;
-  }
+  if (threadIdx.x == 0) pcg_begin_state(mem[blockIdx.x].st, tau);
 }
 
 // after the setup matvec: the n = 0 convergence test and the first beta
@@ -2231,33 +2088,33 @@ int launch_yf_div(const LaunchCtx& c, int s_hx, int s_hy, int s_q, int s_yx, int
 
 template <int L>
 struct RunXfDiv {
-  static int run(const LaunchCtx& c, int mode, int s_yx, int s_rr, int s_p, int s_out) {
-    dim3 g(c.d.n1 * (c.d.m2 / 16), c.nm);
-    const int tb = 2 * CK<L>::TPB, tb3 = 3 * CK<L>::TPB;
-    if (c.xf_split == 2 && mode == XF_MATVEC)
-      k_xf_div_s3<L, XF_MATVEC><<<g, tb3, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
-    else if (c.xf_split == 2 && mode == XF_SETUP)
-      k_xf_div_s3<L, XF_SETUP><<<g, tb3, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
+  // A sum takes the one-group kernel at every length: its two groups would carry one and three of the
+  // five fields (8 x 256^3: 595 us in one group, 650 in two, 711 in three).
+  template <int MODE>
+  static int go(const LaunchCtx& c, int s_yx, int s_rr, int s_rb, int s_p, int s_out) {
+    const dim3 g(c.d.n1 * (c.d.m2 / 16), c.nm);
+    constexpr int tb = CK<L>::TPB;
+    if (s_rb >= 0)
+      k_xf_div<L, MODE, true><<<g, tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_rb, s_p, s_out);
     else if (c.xf_split == 2)
-      k_xf_div_s3<L, XF_D><<<g, tb3, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
-    else if (c.xf_split && mode == XF_MATVEC)
-      k_xf_div_s<L, XF_MATVEC><<<g, tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
-    else if (c.xf_split && mode == XF_SETUP)
-      k_xf_div_s<L, XF_SETUP><<<g, tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
+      k_xf_div_s3<L, MODE><<<g, 3 * tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
     else if (c.xf_split)
-      k_xf_div_s<L, XF_D><<<g, tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
-    else if (mode == XF_MATVEC)
-      k_xf_div<L, XF_MATVEC><<<g, CK<L>::TPB, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
-    else if (mode == XF_SETUP)
-      k_xf_div<L, XF_SETUP><<<g, CK<L>::TPB, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
+      k_xf_div_s<L, MODE><<<g, 2 * tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
     else
-      k_xf_div<L, XF_D><<<g, CK<L>::TPB, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
+      k_xf_div<L, MODE, false><<<g, tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, 0, s_p, s_out);
     GLIA_CHECK_LAUNCH();
     return 0;
   }
+  static int run(const LaunchCtx& c, int mode, int s_yx, int s_rr, int s_rb, int s_p, int s_out) {
+    switch (mode) {
+      case XF_MATVEC: return go<XF_MATVEC>(c, s_yx, s_rr, s_rb, s_p, s_out);
+      case XF_SETUP: return go<XF_SETUP>(c, s_yx, s_rr, s_rb, s_p, s_out);
+      default: return go<XF_D>(c, s_yx, s_rr, s_rb, s_p, s_out);
+    }
+  }
 };
-int launch_xf_div(const LaunchCtx& c, int mode, int s_yx, int s_rr, int s_p, int s_out) {
-  return dispatch_L<RunXfDiv>(c.d.n0, c, mode, s_yx, s_rr, s_p, s_out);
+int launch_xf_div(const LaunchCtx& c, int mode, int s_yx, int s_rr, int s_rb, int s_p, int s_out) {
+  return dispatch_L<RunXfDiv>(c.d.n0, c, mode, s_yx, s_rr, s_rb, s_p, s_out);
 }
 int xf_div_blocks(const Dims& d) { return d.n1 * (d.m2 / 16); }
 

@@ -41,7 +41,14 @@ int ew_blocks();
 int launch_xi_grad(const LaunchCtx& c, int s_in, int s_r, int s_u, int s_v, bool pupd);
 int launch_yi_grad(const LaunchCtx& c, int s_u, int s_v, int s_gx, int s_gy, int s_gz, int s_g0);
 int launch_yf_div(const LaunchCtx& c, int s_hx, int s_hy, int s_q, int s_yx, int s_rr);
-int launch_xf_div(const LaunchCtx& c, int mode, int s_yx, int s_rr, int s_p, int s_out);
+// s_rb >= 0: the second input is the sum of slots s_rr and s_rb
+int launch_xf_div(const LaunchCtx& c, int mode, int s_yx, int s_rr, int s_rb, int s_p, int s_out);
+// the Y and Z passes of the matvec fused over x-planes (plane_kernels.hip): slots U, V -> the x, y and z
+// terms after their forward Y transforms, the y and z terms times i w_y and i w_z.  launch_plane_mask
+// first, with the same k_slot; begin: it also starts a CN solve (as launch_pcg_begin)
+bool plane_supported(const Dims& d);
+int launch_plane_mask(const LaunchCtx& c, int k_slot, bool begin, double tau);
+int launch_plane_diff(const LaunchCtx& c, int s_u, int s_v, int s_x, int s_y, int s_z, int k_slot);
 int launch_col_plain(const LaunchCtx& c, int dir, int sign, int s_in, int s_out, bool honor_done);
 int launch_z_diff(const LaunchCtx& c, int s_gx, int s_gy, int s_gz, int k_slot);
 int launch_z_point(const LaunchCtx& c, int mode, int s_in, int s_out, int r_slot, int ch_idx, float dt, bool honor_done);

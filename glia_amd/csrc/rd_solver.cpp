@@ -119,6 +119,7 @@ int RDEnsemble::init() {
       if (tok == "yfb2") yf_split_ = 3;
     }
   }
+  plane_ = plane_supported(d_);
   if (!supported_line(d_.n0) || !supported_line(d_.n1) || !supported_z(d_.n2))
     return fail(-4, "unsupported grid: n0, n1 in {32,48,64,80,96,128,160,192,256}, n2 in {32,64,96,128,160,192,256}");
   if (z_blocks(d_) <= 0 || ((int64_t)d_.n0 * d_.n1) % z_lines_per_block(d_.m2) != 0)
@@ -223,6 +224,7 @@ int RDEnsemble::alloc_member(int m) {
   nb = std::max<int64_t>(nb, (int64_t)ew_blocks() * 2);
   GLIA_HIP(hipMalloc(&part_[m], sizeof(double) * nb));
   M.part = part_[m];
+  GLIA_HIP(hipMalloc(&M.kmask, sizeof(unsigned) * d_.n0));
   int rc = alloc_history(m);
   if (rc) return rc;
   M.kr_gm = (float)cfg_.k_gm_wm;
@@ -399,6 +401,7 @@ RDEnsemble::~RDEnsemble() {
     free_history(m);
     (void)hipFree(st_[m]);
     (void)hipFree(part_[m]);
+    (void)hipFree(mh_[m].kmask);
     (void)hipFree(bricks_dev_[m]);
     (void)hipFree(brick_data_[m]);
     (void)hipFree(phi_scale_dev_[m]);
@@ -788,14 +791,48 @@ int RDEnsemble::set_spectrum(int m, int cslot, const float2* host) {
   return copy_sync(mh_[m].c[cslot], host, sizeof(float2) * d_.nspec, hipMemcpyHostToDevice);
 }
 
+// the passes of the matvec between its X passes, from U and V in CS_T0 and CS_T1: gradient, product
+// with the real slot k_slot, forward transforms along z and y
+int RDEnsemble::middle_passes(int k_slot, bool timed) {
+  LaunchCtx c = ctx();
+  auto mark = [&](int kind, bool begin) {
+    if (timed) prof_mark(kind, begin);
+  };
+  if (plane_) {
+    mark(PK_PLANE_DIV, true);
+    GLIA_TRYC(launch_plane_diff(c, CS_T0, CS_T1, CS_T2, CS_T3, CS_T4, k_slot));
+    mark(PK_PLANE_DIV, false);
+    return 0;
+  }
+  mark(PK_YI_GRAD, true);
+  GLIA_TRYC(launch_yi_grad(c, CS_T0, CS_T1, CS_T2, CS_T3, CS_T4, -1));
+  mark(PK_YI_GRAD, false);
+  mark(PK_Z_DIFF, true);
+  GLIA_TRYC(launch_z_diff(c, CS_T2, CS_T3, CS_T4, k_slot));
+  mark(PK_Z_DIFF, false);
+  mark(PK_YF_DIV, true);
+  GLIA_TRYC(launch_yf_div(c, CS_T2, CS_T3, CS_T4, CS_T0, CS_T1));
+  mark(PK_YF_DIV, false);
+  return 0;
+}
+
+// the forward X pass after middle_passes
+int RDEnsemble::close_divergence(int mode, int s_p, int s_out) {
+  if (plane_) return launch_xf_div(ctx(), mode, CS_T2, CS_T3, CS_T4, s_p, s_out);
+  return launch_xf_div(ctx(), mode, CS_T0, CS_T1, -1, s_p, s_out);
+}
+
+// the start of a CN solve with the diffusion coefficient RS_K
+int RDEnsemble::solve_begin(double tau) {
+  return plane_ ? launch_plane_mask(ctx(), RS_K, true, tau) : launch_pcg_begin(ctx(), tau);
+}
+
 // b - A x0 for x0 = c: r = tau D c, with the partial norms of B b and B r (KSPConvergedDefault)
 int RDEnsemble::matvec_setup(int sx) {
   LaunchCtx c = ctx();
   GLIA_TRYC(launch_xi_grad(c, sx, 0, CS_T0, CS_T1, false));
-  GLIA_TRYC(launch_yi_grad(c, CS_T0, CS_T1, CS_T2, CS_T3, CS_T4, -1));
-  GLIA_TRYC(launch_z_diff(c, CS_T2, CS_T3, CS_T4, RS_K));
-  GLIA_TRYC(launch_yf_div(c, CS_T2, CS_T3, CS_T4, CS_T0, CS_T1));
-  GLIA_TRYC(launch_xf_div(c, XFM_SETUP, CS_T0, CS_T1, sx, CS_R));
+  GLIA_TRYC(middle_passes(RS_K));
+  GLIA_TRYC(close_divergence(XFM_SETUP, sx, CS_R));
   return 0;
 }
 
@@ -805,7 +842,7 @@ int RDEnsemble::cn_solve(int sx, double tau, int kind) {
   ctx_dt_ = tau;  // ctx->dt_ = dt (src/pde/DiffusionSolver.cpp:226)
   LaunchCtx c = ctx();
   const int nbx = xf_div_blocks(d_);
-  GLIA_TRYC(launch_pcg_begin(c, tau));
+  GLIA_TRYC(solve_begin(tau));
   int rc = matvec_setup(sx);
   if (rc) return rc;
   int stage = 0;
@@ -853,7 +890,7 @@ int RDEnsemble::cn_solve(int sx, double tau, int kind) {
 int RDEnsemble::capture_solve(int sx, double tau, int K, int fslot) {
   ctx_dt_ = tau;
   LaunchCtx c = ctx();
-  GLIA_TRYC(launch_pcg_begin(c, tau));
+  GLIA_TRYC(solve_begin(tau));
   int rc = matvec_setup(sx);
   if (rc) return rc;
   GLIA_TRYC(launch_pcg_fin_setup(c, xf_div_blocks(d_), hflag_dev_, K == 0 ? fslot : 0));
@@ -1051,18 +1088,11 @@ int RDEnsemble::launch_iteration(int sx, int slot) {
   prof_mark(PK_XI_PUPD, true);
   GLIA_TRYC(launch_xi_grad(c, CS_P, CS_R, CS_T0, CS_T1, true));
   prof_mark(PK_XI_PUPD, false);
-  prof_mark(PK_YI_GRAD, true);
-  GLIA_TRYC(launch_yi_grad(c, CS_T0, CS_T1, CS_T2, CS_T3, CS_T4, -1));
-  prof_mark(PK_YI_GRAD, false);
-  prof_mark(PK_Z_DIFF, true);
-  GLIA_TRYC(launch_z_diff(c, CS_T2, CS_T3, CS_T4, RS_K));
-  prof_mark(PK_Z_DIFF, false);
-  prof_mark(PK_YF_DIV, true);
-  GLIA_TRYC(launch_yf_div(c, CS_T2, CS_T3, CS_T4, CS_T0, CS_T1));
-  prof_mark(PK_YF_DIV, false);
-  prof_mark(PK_XF_MATVEC, true);
-  GLIA_TRYC(launch_xf_div(c, XFM_MATVEC, CS_T0, CS_T1, CS_P, CS_W));
-  prof_mark(PK_XF_MATVEC, false);
+  int rc = middle_passes(RS_K, true);
+  if (rc) return rc;
+  prof_mark(plane_ ? PK_XF_SUM : PK_XF_MATVEC, true);
+  GLIA_TRYC(close_divergence(XFM_MATVEC, CS_P, CS_W));
+  prof_mark(plane_ ? PK_XF_SUM : PK_XF_MATVEC, false);
   GLIA_TRYC(launch_pcg_fin_dpi(c, nbx));
   prof_mark(PK_PCG_UPDATE, true);
   GLIA_TRYC(launch_pcg_update(c, sx));
@@ -1282,11 +1312,10 @@ int RDEnsemble::apply_dsec(int in, int out) {
   int rc = clear_done();
   if (rc) return rc;
   LaunchCtx c = ctx();
+  if (plane_) GLIA_TRYC(launch_plane_mask(c, RS_KS, false, 0.0));
   GLIA_TRYC(launch_xi_grad(c, in, 0, CS_T0, CS_T1, false));
-  GLIA_TRYC(launch_yi_grad(c, CS_T0, CS_T1, CS_T2, CS_T3, CS_T4, -1));
-  GLIA_TRYC(launch_z_diff(c, CS_T2, CS_T3, CS_T4, RS_KS));
-  GLIA_TRYC(launch_yf_div(c, CS_T2, CS_T3, CS_T4, CS_T0, CS_T1));
-  GLIA_TRYC(launch_xf_div(c, XFM_D, CS_T0, CS_T1, in, out));
+  GLIA_TRYC(middle_passes(RS_KS));
+  GLIA_TRYC(close_divergence(XFM_D, in, out));
   return 0;
 }
 
@@ -1584,7 +1613,7 @@ int RDEnsemble::autotune(const char* cache_path, int* choice) {
   double xf_ms[kXfVariants], yf_ms[kYfVariants];
   for (int v = 0; v < kXfVariants && !rc; v++) {
     xf_split_ = v;
-    rc = time_it([&]() { return launch_xf_div(ctx(), XFM_MATVEC, CS_T0, CS_T1, CS_P, CS_W); }, &xf_ms[v]);
+    rc = time_it([&]() { return close_divergence(XFM_MATVEC, CS_P, CS_W); }, &xf_ms[v]);
   }
   for (int v = 0; v < kYfVariants && !rc; v++) {
     yf_split_ = v;
@@ -1669,11 +1698,10 @@ int RDEnsemble::apply_d_field(int rin, int rout) {
   rc = clear_done();
   if (rc) return rc;
   LaunchCtx c = ctx();
+  if (plane_) GLIA_TRYC(launch_plane_mask(c, RS_K, false, 0.0));
   GLIA_TRYC(launch_xi_grad(c, CS_X, 0, CS_T0, CS_T1, false));
-  GLIA_TRYC(launch_yi_grad(c, CS_T0, CS_T1, CS_T2, CS_T3, CS_T4, -1));
-  GLIA_TRYC(launch_z_diff(c, CS_T2, CS_T3, CS_T4, RS_K));
-  GLIA_TRYC(launch_yf_div(c, CS_T2, CS_T3, CS_T4, CS_T0, CS_T1));
-  GLIA_TRYC(launch_xf_div(c, XFM_D, CS_T0, CS_T1, CS_X, CS_T5));
+  GLIA_TRYC(middle_passes(RS_K));
+  GLIA_TRYC(close_divergence(XFM_D, CS_X, CS_T5));
   rc = inverse_to_real(CS_T5, CS_T6, rout);
   if (rc) return rc;
   return sync();

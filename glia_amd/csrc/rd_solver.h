@@ -34,7 +34,8 @@ struct SolverConfig {
 };
 
 // kernel kinds timed by the profiling mode (HIP events around each launch on the solver stream)
-enum ProfKind { PK_XI_PUPD = 0, PK_YI_GRAD, PK_Z_DIFF, PK_YF_DIV, PK_XF_MATVEC, PK_PCG_UPDATE, PK_NUM };
+enum ProfKind { PK_XI_PUPD = 0, PK_YI_GRAD, PK_Z_DIFF, PK_YF_DIV, PK_XF_MATVEC, PK_PCG_UPDATE, PK_PLANE_DIV, PK_XF_SUM,
+                PK_NUM };
 
 struct MemberStats {
   int its_total, solves, worst_reason, last_its, last_reason;
@@ -232,6 +233,9 @@ class RDEnsemble {
   int adjoint_step_stored(int i);
   int launch_iteration(int sx, int slot);                       // the launches of one CG iteration
   int iteration_graph(int sx, int slot, hipGraphExec_t* out);   // the same, captured once and cached
+  int middle_passes(int k_slot, bool timed = false);
+  int close_divergence(int mode, int s_p, int s_out);
+  int solve_begin(double tau);
   int matvec_setup(int sx);
   int forward_step(int sx, int step, bool store_half);
   int forward_transform_real(int rslot, int cslot);  // R2C of a real slot into a complex slot
@@ -311,6 +315,7 @@ class RDEnsemble {
     int kind;
     hipEvent_t a, b;
   };
+  bool plane_ = false;  // Y and Z passes of the matvec fused over x-planes
   int yf_split_ = 0, xf_split_ = 0;  // variants of the forward divergence passes (autotune)
   static constexpr int kYfVariants = 4;
   static constexpr int kXfVariants = 3;
