@@ -285,6 +285,8 @@ int RDEnsemble::set_time(double dt, int nt) {
   GLIA_HIP(hipStreamSynchronize(stream_));
   cfg_.dt = dt;
   if (nt == cfg_.nt) return 0;
+  for (auto& sw : step_its_)
+    for (auto& k : sw) k.clear();
   for (int m = 0; m < nm_; m++) free_history(m);
   cfg_.nt = nt;
   npool_ = hist_all_ ? cfg_.nt + 1 : std::max(1, cfg_.checkpoint_slots);
@@ -958,17 +960,40 @@ int RDEnsemble::read_step_flags(int nsolve, int* its, bool* ok) {
   return 0;
 }
 
+// Iteration budget of a solve of time step i (-1: run the step eagerly), before the margin: the count
+// the same solve of the same step had in the last evaluation, plus what the step before exceeded its own
+// by in this one.  Without one, small grids take the count of the last solve of the kind.  On large ones
+// the step runs eagerly instead: a wrong budget costs the whole step again, while launches from the host
+// cost nothing there (a kernel at 2 x 128^3 takes 12 us, its launch 4).  With the last solve's count
+// throughout, steps whose counts differ ran twice: 8 x 256^3 at nt = 2 453 ms an evaluation against 313
+// ms eagerly.
+int RDEnsemble::step_budget(int kind, int i, bool first) const {
+  const auto& own = step_its_[sweep_][kind];
+  if (i < (int)own.size() && own[i] >= 0) return own[i] + (first ? 0 : std::max(0, drift_[kind]));
+  return (int64_t)nm_ * d_.ng >= ((int64_t)1 << 22) ? -1 : budget_[kind];
+}
+
+void RDEnsemble::step_done(int kind, int i, int its, bool first) {
+  auto& own = step_its_[sweep_][kind];
+  if ((int)own.size() != cfg_.nt) own.assign(cfg_.nt, -1);
+  if (first) drift_[kind] = 0;
+  if (own[i] >= 0) drift_[kind] = its - own[i];
+  own[i] = its;
+  budget_[kind] = its;
+}
+
 // one forward Strang step (forward_step) from c_i in CS_X, with c_{i+1} stored in the history:
-// replayed from a graph captured with iteration budgets one above (margin_) the last solves' counts; when
+// replayed from a graph captured with iteration budgets one above (margin_) step_budget's counts; when
 // a solve needs more, the counters return to the step's start and the step runs again eagerly
 // from c_i (stored in the history), so the result is that of forward_step.  fwd_prepare gives the
 // step's graph (null when the step runs eagerly: no budgets yet, or graphs off); fwd_finish runs
 // after its launch, or in place of it.
 int RDEnsemble::fwd_prepare(int i, bool store_half, const StepGraph** out) {
   *out = nullptr;
-  if (!(step_graphs_on() && budget_[SK_FWD1] >= 0 && budget_[SK_FWD2] >= 0)) return 0;
+  const int b1 = step_budget(SK_FWD1, i, i == 0), b2 = step_budget(SK_FWD2, i, i == 0);
+  if (!(step_graphs_on() && b1 >= 0 && b2 >= 0)) return 0;
   const double dt = cfg_.dt;
-  const int K1 = std::max(0, budget_[SK_FWD1] + margin_), K2 = std::max(0, budget_[SK_FWD2] + margin_);
+  const int K1 = std::max(0, b1 + margin_), K2 = std::max(0, b2 + margin_);
   const StepKey key{0, i, K1, K2, 0, store_half ? 1 : 0};
   return step_graph(key, [&]() -> int {
     LaunchCtx c = ctx();
@@ -994,8 +1019,8 @@ int RDEnsemble::fwd_finish(int i, bool store_half, bool launched) {
     bool ok = false;
     if ((rc = read_step_flags(2, its, &ok))) return rc;
     if (ok) {
-      budget_[SK_FWD1] = its[0];
-      budget_[SK_FWD2] = its[1];
+      step_done(SK_FWD1, i, its[0], i == 0);
+      step_done(SK_FWD2, i, its[1], i == 0);
       return 0;
     }
     step_reruns_++;
@@ -1003,6 +1028,8 @@ int RDEnsemble::fwd_finish(int i, bool store_half, bool launched) {
     GLIA_TRYC(launch_copy(ctx(), state_slot(i), CS_X));
   }
   if ((rc = forward_step(CS_X, i, store_half))) return rc;
+  step_done(SK_FWD1, i, budget_[SK_FWD1], i == 0);
+  step_done(SK_FWD2, i, budget_[SK_FWD2], i == 0);
   GLIA_TRYC(launch_copy(ctx(), CS_X, state_slot(i + 1)));
   return 0;
 }
@@ -1020,11 +1047,13 @@ int RDEnsemble::forward_step_stored(int i, bool store_half) {
 int RDEnsemble::adj_prepare(int i, const StepGraph** out) {
   *out = nullptr;
   const bool half = cfg_.adjoint_store != 0;  // c_half_ stored, no recomputation solve
-  if (!(step_graphs_on() && budget_[SK_ADJ1] >= 0 && budget_[SK_ADJ2] >= 0 && (half || budget_[SK_HALF] >= 0)))
-    return 0;
+  const bool first = i == cfg_.nt - 1;
+  const int b1 = step_budget(SK_ADJ1, i, first), b2 = step_budget(SK_ADJ2, i, first);
+  const int bh = half ? 0 : step_budget(SK_HALF, i, first);
+  if (!(step_graphs_on() && b1 >= 0 && b2 >= 0 && bh >= 0)) return 0;
   const double dt = cfg_.dt;
-  const int K1 = std::max(0, budget_[SK_ADJ1] + margin_), K2 = std::max(0, budget_[SK_ADJ2] + margin_);
-  const int Kh = half ? 0 : std::max(0, budget_[SK_HALF] + margin_);
+  const int K1 = std::max(0, b1 + margin_), K2 = std::max(0, b2 + margin_);
+  const int Kh = half ? 0 : std::max(0, bh + margin_);
   const int flags = (half ? 1 : 0) | (quad_on_ ? 2 : 0) | (keep_adj_ ? 4 : 0);
   const StepKey key{1, i, K1, K2, Kh, flags};
   return step_graph(key, [&]() -> int {
@@ -1050,24 +1079,29 @@ int RDEnsemble::adj_prepare(int i, const StepGraph** out) {
 }
 
 int RDEnsemble::adj_finish(int i, bool launched) {
+  const bool half = cfg_.adjoint_store != 0, first = i == cfg_.nt - 1;
   if (launched) {
     step_launches_++;
-    const bool half = cfg_.adjoint_store != 0;
     int its[3] = {0, 0, 0};
     bool ok = false;
     int rc = read_step_flags(half ? 2 : 3, its, &ok);
     if (rc) return rc;
     if (ok) {
-      budget_[SK_ADJ1] = its[0];
-      budget_[SK_ADJ2] = its[1];
-      if (!half) budget_[SK_HALF] = its[2];
+      step_done(SK_ADJ1, i, its[0], first);
+      step_done(SK_ADJ2, i, its[1], first);
+      if (!half) step_done(SK_HALF, i, its[2], first);
       return 0;
     }
     step_reruns_++;
     GLIA_TRYC(launch_state_reset(ctx(), 8));
     GLIA_TRYC(launch_copy(ctx(), CS_BK, CS_A));
   }
-  return adjoint_step(i, state_slot(i));
+  const int rc = adjoint_step(i, state_slot(i));
+  if (rc) return rc;
+  step_done(SK_ADJ1, i, budget_[SK_ADJ1], first);
+  step_done(SK_ADJ2, i, budget_[SK_ADJ2], first);
+  if (!half) step_done(SK_HALF, i, budget_[SK_HALF], first);
+  return 0;
 }
 
 int RDEnsemble::adjoint_step_stored(int i) {
@@ -1373,6 +1407,7 @@ int RDEnsemble::incremental_adjoint(int ct_slot, bool quads) {
   GLIA_TRYC(launch_col_plain(c, 1, -1, CS_T5, CS_T5, false));
   GLIA_TRYC(launch_col_plain(c, 0, -1, CS_T5, CS_A, false));
   quad_on_ = quads;
+  sweep_ = 1;
   rc = 0;
   if (hist_all_) {
     for (int i = cfg_.nt - 1; i >= 0 && rc == 0; i--) rc = adjoint_step_stored(i);
@@ -1380,6 +1415,7 @@ int RDEnsemble::incremental_adjoint(int ct_slot, bool quads) {
     rc = reverse(0, cfg_.nt, stored_[0], npool_ - 1);
   }
   quad_on_ = true;
+  sweep_ = 0;
   if (rc) return rc;
   return inverse_to_real(CS_A, CS_T5, RS_A0);
 }

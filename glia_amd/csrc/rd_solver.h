@@ -294,6 +294,13 @@ class RDEnsemble {
   static constexpr int kStepFlags = 3;  // host flag slots of the budgeted solves of a captured step
   hipEvent_t ev_step_ = nullptr;
   int budget_[SK_NUM] = {-1, -1, -1, -1, -1};  // iterations of the last solve of each kind (-1: none yet)
+  // iterations of each solve of each time step in the last evaluation that ran it, per sweep (0: forward
+  // and gradient adjoint, 1: incremental adjoint), and how far the last step exceeded its own
+  std::vector<int> step_its_[2][SK_NUM];
+  int drift_[SK_NUM] = {0, 0, 0, 0, 0};
+  int sweep_ = 0;
+  int step_budget(int kind, int i, bool first) const;
+  void step_done(int kind, int i, int its, bool first);
   std::map<StepKey, StepGraph> step_graphs_;
   long long step_reruns_ = 0;  // captured steps that ran again eagerly
   long long step_launches_ = 0;  // captured steps launched
