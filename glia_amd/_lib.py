@@ -294,8 +294,8 @@ ME_SIGNATURES = {
 
 KERNELS = ["xi_pupd", "yi_grad", "z_diff", "yf_div", "xf_matvec", "pcg_update", "plane_div", "xf_sum"]
 # algorithmic bytes of one launch per member, in units of one field (4 n0 n1 n2 bytes): every
-# input read once and every output written once.  Grids with n1 = n2 run plane_div and xf_sum in place
-# of yi_grad, z_diff, yf_div and xf_matvec; plane_div does not read or transform planes where k is zero
+# input read once and every output written once.  Grids with n1 and n2 within a factor of two run
+# plane_div and xf_sum in place of yi_grad, z_diff, yf_div and xf_matvec; plane_div does not read or transform planes where k is zero
 KERNEL_FIELDS = {"xi_pupd": 5, "yi_grad": 5, "z_diff": 7, "yf_div": 5, "xf_matvec": 4, "pcg_update": 6,
                  "plane_div": 6, "xf_sum": 5}
 

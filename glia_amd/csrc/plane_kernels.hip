@@ -14,10 +14,12 @@
 // rows without block barriers.
 //
 // What bounds it: at 128 points the vector units (about 4200 instructions a lane and component, 65% of
-// the issue slots; two blocks a CU).  From 160 points one block fits a CU (registers), so a block's
-// loads and stores are not covered by another's arithmetic.  Measured against the three passes it
+// the issue slots; two blocks a CU).  From 160 points a CU holds ten or fewer waves (registers), too
+// few to cover a block's loads and stores with arithmetic.  Measured against the three passes it
 // replaces, matvec middle of one CG iteration with every member active: 16 x 128^3 450 -> 193 us,
-// 8 x 160^3 424 -> 285, 8 x 192^3 726 -> 442, 8 x 256^3 1761 -> 882 (17 fields of traffic became 6).
+// 8 x 160^3 424 -> 252, 8 x 192^3 726 -> 442, 8 x 256^3 1761 -> 882 (17 fields of traffic became 6).
+// Whole CN solves of four members on 96 x n1 x n2 grids: 1.05 to 1.35 times as fast at every size built
+// (96 x 96 1.38 -> 1.02 ms, 160 x 96 1.99 -> 1.74, 192 x 128 3.18 -> 2.83, 256 x 160 6.47 -> 6.17).
 #include <hip/hip_runtime.h>
 
 #include "lane_fft.h"
@@ -32,14 +34,22 @@ template <int N1, int N2>
 struct PL {
   static constexpr int M = N2 / 2;
   static constexpr int RY = N1 / 4, RZ = M / 2, H = RZ / 2;  // values per lane in the two layouts
-  static constexpr int WY = M / 16, WZ = N1 / 32;            // waves that hold them
-  static constexpr int W = WY > WZ ? WY : WZ, T = 64 * W;
+  static constexpr int WY = M / 16, WZ = (N1 + 31) / 32;     // waves that hold them
+  static constexpr int W = WY > WZ ? WY : WZ, T = 64 * W;  // waves and threads of one plane
   // row pitch of the plane in LDS, odd so that 32 lanes on 32 lines hit distinct banks; 17 mod 64 at
   // M = 128 keeps the 4 x 16 column accesses of the Y layout apart too
   static constexpr int P = M == 128 ? 145 : M + 1;
   // planes that would leave room for one block only are turned in two halves (real, then imaginary)
   static constexpr bool SPLIT = N1 * P * 8 > 76 * 1024;
-  static constexpr int LDS = N1 * P * (SPLIT ? 1 : 2);  // floats
+  static constexpr int LDS = 32 * WZ * P * (SPLIT ? 1 : 2);  // floats
+  static constexpr int LINES = N1;
+  // Planes of 5 to 7 waves go two to a block.  As blocks of their own only one would run on a CU: a
+  // block's waves are dealt to the SIMDs from the first one on, so a second block of 5 waves would put
+  // four on that SIMD, which their registers do not allow; ten waves of one block put three there (8 x
+  // 160^3: 285 -> 252 us).  With more than 40 values a lane three waves a SIMD spill, and one plane a
+  // block is the better one (192 x 128: 3.25 -> 2.83 ms a solve; 192 x 192 alike).
+  static constexpr int CH = W > 4 && W < 8 && RY <= 40 && RZ <= 40 ? 2 : 1;
+  static constexpr int TB = CH * T, MINW = CH == 2 ? 3 : 2;
 };
 
 __device__ __forceinline__ void wave_fence() {
@@ -60,7 +70,7 @@ struct PlaneLane {
 };
 template <class K>
 __device__ __forceinline__ PlaneLane plane_lane() {
-  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  const int lane = (int)threadIdx.x & 63, wave = ((int)threadIdx.x >> 6) % K::W;
   PlaneLane L;
   L.yc = wave * 16 + (lane & 15);
   L.yt = lane >> 4;
@@ -125,7 +135,7 @@ __device__ __forceinline__ void y_write(float* lds, const PlaneLane& L, unsigned
   for (int g = 0; g < K::WZ; g++) {
     if (!(mask >> g & 1)) continue;
 #pragma unroll
-    for (int j = 8 * g; j < 8 * g + 8; j++) {
+    for (int j = 8 * g; j < (8 * g + 8 < K::RY ? 8 * g + 8 : K::RY); j++) {
       const int i = L.yt * K::P + L.yc + 4 * j * K::P;
       if constexpr (!K::SPLIT)
         reinterpret_cast<float2*>(lds)[i] = v[j];
@@ -140,7 +150,7 @@ __device__ __forceinline__ void y_read(const float* lds, const PlaneLane& L, uns
   for (int g = 0; g < K::WZ; g++) {
     const bool on = mask >> g & 1;
 #pragma unroll
-    for (int j = 8 * g; j < 8 * g + 8; j++) {
+    for (int j = 8 * g; j < (8 * g + 8 < K::RY ? 8 * g + 8 : K::RY); j++) {
       const int i = L.yt * K::P + L.yc + 4 * j * K::P;
       if constexpr (!K::SPLIT)
         v[j] = on ? reinterpret_cast<const float2*>(lds)[i] : make_float2(0.0f, 0.0f);
@@ -248,8 +258,8 @@ __device__ __forceinline__ float y_wave(int j, int t) {
 template <class K, int N1>
 __device__ __forceinline__ void stage_plane_twiddles(float2* ty, float2* tm, float2* t2, const float2* __restrict__ tw1,
                                                      const float2* __restrict__ twm, const float2* __restrict__ tw2) {
-  for (int i = threadIdx.x; i < N1; i += K::T) ty[i] = tw1[(i & 3) * (i >> 2)];
-  for (int i = threadIdx.x; i < K::M; i += K::T) {
+  for (int i = threadIdx.x; i < N1; i += K::TB) ty[i] = tw1[(i & 3) * (i >> 2)];
+  for (int i = threadIdx.x; i < K::M; i += K::TB) {
     tm[i] = twm[(i & 1) * (i >> 1)];
     t2[i] = tw2[i];
   }
@@ -269,15 +279,17 @@ template <class K, int PART, int HP>
 __device__ __forceinline__ void real_fetch(float2 (&q)[RealPart<K>::CNT], GPtrT<HP> field, const PlaneLane& L) {
   using RP = RealPart<K>;
   const int lane = (int)threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(L.zl >> 5);
   const auto f0 = field + (wave * 32 * K::M + PART * RP::PM);
 #pragma unroll
   for (int i = 0; i < RP::CNT; i++) {
-    if constexpr (RP::PARTS == 1) {  // the wave's lines are one run
+    const unsigned e = (unsigned)(i * 64 + lane), row = e / RP::PM;
+    if (K::LINES % 32 != 0 && wave * 32 + (int)row >= K::LINES) {
+      q[i] = make_float2(0.0f, 0.0f);
+    } else if constexpr (RP::PARTS == 1) {  // the wave's lines are one run
       q[i] = (f0 + i * 64)[(unsigned)lane];
     } else {
-      const unsigned e = (unsigned)(i * 64 + lane);
-      q[i] = f0[(e / RP::PM) * K::M + e % RP::PM];
+      q[i] = f0[row * K::M + e % RP::PM];
     }
   }
 }
@@ -344,13 +356,14 @@ __global__ void __launch_bounds__(256) k_plane_mask(const MemberDev* __restrict_
                                                     double tau) {
   const MemberDev& M = mem[blockIdx.y];
   if (begin && blockIdx.x == 0 && threadIdx.x == 0) pcg_begin_state(M.st, tau);
-  const unsigned n4 = (unsigned)(32 * d.n2 / 4);  // 16-byte words of a group
+  const unsigned n4 = (unsigned)(32 * d.n2 / 4), all = (unsigned)(d.n1 * d.n2 / 4);  // 16-byte words: group, plane
   const v4f* f = reinterpret_cast<const v4f*>(M.r[k_slot] + (int64_t)blockIdx.x * d.n1 * d.n2);
   unsigned mask = 0;
-  for (int g = 0; g < d.n1 / 32; g++) {
+  for (int g = 0; 32 * g < d.n1; g++) {
     int any = 0;
-    for (unsigned i = threadIdx.x; i < n4; i += 256) {
-      const v4f x = f[g * n4 + i];
+    const unsigned end = (g + 1) * n4 < all ? (g + 1) * n4 : all;
+    for (unsigned i = g * n4 + threadIdx.x; i < end; i += 256) {
+      const v4f x = f[i];
       any |= !(x.x == 0.0f && x.y == 0.0f && x.z == 0.0f && x.w == 0.0f);
     }
     if (__syncthreads_or(any)) mask |= 1u << g;
@@ -365,25 +378,30 @@ __global__ void __launch_bounds__(256) k_plane_mask(const MemberDev* __restrict_
 // One block per plane and component, the three components of a plane on one XCD (blocks go to the 8
 // XCDs round-robin), which share the k and U planes in its L2.
 template <int N1, int N2>
-__global__ void __launch_bounds__((PL<N1, N2>::T), 2)
+__global__ void __launch_bounds__((PL<N1, N2>::TB), (PL<N1, N2>::MINW))
 k_plane_diff(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ tw1, const float2* __restrict__ twm,
              const float2* __restrict__ tw2, int s_u, int s_v, int s_x, int s_y, int s_z, int k_slot) {
   using K = PL<N1, N2>;
   using RP = RealPart<K>;
   const MemberDev& Mb = mem[blockIdx.y];
   if (Mb.st->done) return;
-  __shared__ float lds[K::LDS];
+  __shared__ float lds_[K::CH][K::LDS];
   __shared__ float2 ty[N1], tm[K::M], t2[K::M];
+  // eight plane groups (one per XCD) times three components, CH planes a group
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), ch = wave / K::W;
   const int q = (int)blockIdx.x >> 3;
-  const int comp = q % 3, plane = (q / 3) * 8 + ((int)blockIdx.x & 7);
+  const int comp = q % 3, plane = ((q / 3) * 8 + ((int)blockIdx.x & 7)) * K::CH + ch;
+  float* lds = lds_[ch];
   const unsigned mask = (unsigned)__builtin_amdgcn_readfirstlane((int)Mb.kmask[plane]);
-  const bool z_on = mask >> __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) & 1;
+  const bool z_on = mask >> (wave - ch * K::W) & 1;
   const int64_t base = (int64_t)plane * N1 * K::M;
   const auto in = uniform(cptr<0>(Mb, comp == 0 ? s_v : s_u) + base);
   const auto out = uniform(cptr<0>(Mb, comp == 0 ? s_x : (comp == 1 ? s_y : s_z)) + base);
   const auto kf = uniform(rptr2<0>(Mb, k_slot) + base);
   PlaneLane L = plane_lane<K>();
-  if (mask == 0) {
+  // nothing to transform (the block's other plane, if any, included: with one plane to do, the other's
+  // rows read as zero below and give zeros)
+  if (mask == 0 && (K::CH == 1 || Mb.kmask[plane ^ 1] == 0)) {
     if (L.y_on) {
 #pragma unroll 4
       for (int j = 0; j < K::RY; j++) (out + 4 * j * K::M)[(unsigned)(L.yt * K::M + L.yc)] = make_float2(0.0f, 0.0f);
@@ -448,30 +466,38 @@ k_plane_diff(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict
 // ---------------------------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------------------------
+// The plane sizes built: sides within a factor of two.  Beyond that most of a block's waves would sit
+// idle in one of the layouts (at 256 x 64, two of eight waves hold the columns).
+#define GLIA_PLANES(X)                                                                        \
+  X(32, 32) X(32, 64) X(48, 32) X(48, 64) X(48, 96) X(64, 32) X(64, 64) X(64, 96) X(64, 128)  \
+  X(80, 64) X(80, 96) X(80, 128) X(80, 160) X(96, 64) X(96, 96) X(96, 128) X(96, 160) X(96, 192) \
+  X(128, 64) X(128, 96) X(128, 128) X(128, 160) X(128, 192) X(128, 256)                       \
+  X(160, 96) X(160, 128) X(160, 160) X(160, 192) X(160, 256)                                  \
+  X(192, 96) X(192, 128) X(192, 160) X(192, 192) X(192, 256)                                  \
+  X(256, 128) X(256, 160) X(256, 192) X(256, 256)
+
 template <template <int, int> class F, typename... Args>
 static int dispatch_plane(const Dims& d, Args&&... args) {
-  if (d.n1 != d.n2) return -1;
-  switch (d.n1) {
-    case 32: return F<32, 32>::run(args...);
-    case 64: return F<64, 64>::run(args...);
-    case 96: return F<96, 96>::run(args...);
-    case 128: return F<128, 128>::run(args...);
-    case 160: return F<160, 160>::run(args...);
-    case 192: return F<192, 192>::run(args...);
-    case 256: return F<256, 256>::run(args...);
-    default: return -1;
-  }
+#define GLIA_PLANE_CASE(A, B) \
+  if (d.n1 == A && d.n2 == B) return F<A, B>::run(args...);
+  GLIA_PLANES(GLIA_PLANE_CASE)
+#undef GLIA_PLANE_CASE
+  return -1;
 }
 
 bool plane_supported(const Dims& d) {
-  return d.n1 == d.n2 && d.n0 % 8 == 0 &&
-         (d.n1 == 32 || d.n1 == 64 || d.n1 == 96 || d.n1 == 128 || d.n1 == 160 || d.n1 == 192 || d.n1 == 256);
+  if (d.n0 % 16 != 0) return false;
+#define GLIA_PLANE_CASE(A, B) \
+  if (d.n1 == A && d.n2 == B) return true;
+  GLIA_PLANES(GLIA_PLANE_CASE)
+#undef GLIA_PLANE_CASE
+  return false;
 }
 
 template <int N1, int N2>
 struct RunPlaneDiff {
   static int run(const LaunchCtx& c, int s_u, int s_v, int s_x, int s_y, int s_z, int k_slot) {
-    k_plane_diff<N1, N2><<<dim3(3 * c.d.n0, c.nm), PL<N1, N2>::T, 0, c.stream>>>(c.mem, c.d, c.tw1, c.twm, c.tw2, s_u, s_v,
+    k_plane_diff<N1, N2><<<dim3(3 * c.d.n0 / PL<N1, N2>::CH, c.nm), PL<N1, N2>::TB, 0, c.stream>>>(c.mem, c.d, c.tw1, c.twm, c.tw2, s_u, s_v,
                                                                               s_x, s_y, s_z, k_slot);
     return (int)hipGetLastError();
   }

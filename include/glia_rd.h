@@ -294,8 +294,8 @@ enum {
   GLIA_RD_K_YF_DIV = 3,    /* Y pass: forward, partial divergence */
   GLIA_RD_K_XF_MATVEC = 4, /* X pass: forward, w = p - tau/2 D p, <p, w> */
   GLIA_RD_K_PCG_UPDATE = 5, /* x, r update with ||B r||^2 and <B r, r> */
-  GLIA_RD_K_PLANE_DIV = 6, /* n1 = n2: kinds 1 to 3 fused over x-planes */
-  GLIA_RD_K_XF_SUM = 7     /* n1 = n2: kind 4 with its second input in two parts */
+  GLIA_RD_K_PLANE_DIV = 6, /* kinds 1 to 3 fused over x-planes (n1 and n2 within a factor of two) */
+  GLIA_RD_K_XF_SUM = 7     /* kind 4 after kind 6, its second input in two parts */
 };
 /* Replay each CG iteration from a captured HIP graph (default on; one graph per solved slot and
    flag slot, built on first use).  Profiling runs always launch kernel by kernel.  No reference
@@ -310,8 +310,8 @@ int glia_rd_use_graphs(glia_rd_t h, int enable);
    cache_path (may be NULL) names a text
    file of earlier choices, read first and appended to.  choice (2 ints, may be NULL) receives
    (X-pass variant, Y-pass variant).  Call before the first solve; the results do not change
-   beyond FP32 rounding.  On grids with n1 = n2 the diffusion operator runs its Y and Z passes fused
-   and these variants are not on its path. */
+   beyond FP32 rounding.  On grids with n1 and n2 within a factor of two the diffusion operator runs
+   its Y and Z passes fused and these variants are not on its path. */
 int glia_rd_autotune(glia_rd_t h, const char* cache_path, int* choice);
 /* Time steps replayed from captured graphs (glia_rd_use_graphs on, store-all history): each
    forward and adjoint step runs as one graph whose CG loops are unrolled to the last iteration

@@ -1,5 +1,6 @@
-"""The plane pass of the diffusion operator (grids with n1 = n2) against an FP64 FFT on the CPU: every
-built plane size, with a coefficient that vanishes on whole planes, on whole groups of 32 lines and on
+"""The plane pass of the diffusion operator against an FP64 FFT on the CPU: every square size and
+rectangular ones (lines that do not fill a wave, more waves in one layout than in the other, two planes
+a block), with a coefficient that vanishes on whole planes, on whole groups of 32 lines and on
 parts of a group, and one that vanishes nowhere."""
 import numpy as np
 import pytest
@@ -32,8 +33,9 @@ def fields(n, kind, rng):
 
 @pytest.mark.parametrize("kind", ["dense", "sparse"])
 @pytest.mark.parametrize("n", [(32, 32, 32), (48, 64, 64), (32, 96, 96), (80, 128, 128), (32, 160, 160), (32, 192, 192),
-                               (32, 256, 256)])
-def test_operator_on_square_planes(n, kind):
+                               (32, 256, 256), (32, 48, 64), (48, 80, 160), (32, 96, 64), (32, 96, 192),
+                               (32, 128, 256), (32, 160, 128), (32, 192, 96), (32, 256, 192)])
+def test_operator_on_planes(n, kind):
     from glia_amd import rd
     print("case plane", n, kind, flush=True)
     rng = np.random.default_rng([n[0], n[1], kind == "sparse"])
