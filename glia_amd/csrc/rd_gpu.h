@@ -163,4 +163,27 @@ __device__ __forceinline__ void pcg_begin_state(PcgState* s, double tau) {
   }
 }
 
+// the vector update of an elasticity CG iteration, from its state and, for the x and r update, the
+// summed <p, A p>: p = z + t p with t = beta / betaold (upd false: p = z, the first iteration and a
+// zero beta), or x += t p, r -= t w with t = beta / <p, A p> (upd false: none, where the CG stops on
+// <p, A p>: 0, not finite, or of the sign opposite to the last one's after the first iteration)
+struct CgStep {
+  float t;
+  bool upd;
+};
+template <bool XR>
+__device__ __forceinline__ CgStep cg_step(const PcgState* S, const double* sc) {
+  CgStep c{0.0f, false};
+  if (XR) {
+    const double q = sc[0];
+    c.upd = !(isnan(q) || isinf(q) || q == 0.0 || (S->i != 0 && q * S->dpi <= 0.0));
+    if (c.upd) c.t = (float)(S->beta / q);
+  } else {
+    const double b = S->i ? S->beta / S->betaold : 0.0;
+    c.upd = b != 0.0;
+    c.t = (float)b;
+  }
+  return c;
+}
+
 }  // namespace glia

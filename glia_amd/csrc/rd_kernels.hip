@@ -1152,17 +1152,9 @@ k_z_upd_r2c(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict_
   const int li = threadIdx.x / NT, t = threadIdx.x % NT;
   const int64_t base = (int64_t)blockIdx.x * ZK<M>::NL * M;
   float2* line = lb + li * ZK<M>::LP;
-  float cf = 0.0f;
-  bool upd = true;
-  double beta = 0.0;
-  if (MODE == ZU_AXPBY) {
-    beta = S->i ? S->beta / S->betaold : 0.0;
-    cf = (float)beta;
-  } else {
-    const double q = sc[0], dpiold = S->dpi;
-    upd = !(isnan(q) || isinf(q) || q == 0.0 || (S->i != 0 && q * dpiold <= 0.0));
-    if (upd) cf = (float)(S->beta / q);
-  }
+  const CgStep cg = cg_step<MODE == ZU_CGUPD>(S, sc);
+  const float cf = cg.t;
+  const bool upd = cg.upd;
   GPtrT<H> A = rptr2<H>(Mb, ra) + base, B = rptr2<H>(Mb, rb) + base;
   float2 tmp[IT];
   if (MODE == ZU_AXPBY) {
@@ -1170,12 +1162,12 @@ k_z_upd_r2c(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict_
 #pragma unroll
     for (int i = 0; i < IT; i++) {
       za[i] = B[(int)threadIdx.x + i * TPB];
-      if (beta != 0.0) pa[i] = A[(int)threadIdx.x + i * TPB];
+      if (upd) pa[i] = A[(int)threadIdx.x + i * TPB];
     }
 #pragma unroll
     for (int i = 0; i < IT; i++) {
       float2 v = za[i];
-      if (beta != 0.0) v = make_float2(za[i].x + cf * pa[i].x, za[i].y + cf * pa[i].y);
+      if (upd) v = make_float2(za[i].x + cf * pa[i].x, za[i].y + cf * pa[i].y);
       A[(int)threadIdx.x + i * TPB] = v;
       tmp[i] = v;
     }
@@ -2427,8 +2419,8 @@ int launch_lane_lin(const LaunchCtx& c, const int* nterms, const int (*lane)[4],
   return 0;
 }
 
-int launch_lane_part_sum(const LaunchCtx& c, int nq, double* out) {
-  k_lane_part_sum<<<1, 256, 0, c.stream>>>(c.mem, c.nm, z_blocks(c.d), nq, out);
+int launch_lane_part_sum(const LaunchCtx& c, int nb, int nq, double* out) {
+  k_lane_part_sum<<<1, 256, 0, c.stream>>>(c.mem, c.nm, nb, nq, out);
   GLIA_CHECK_LAUNCH();
   return 0;
 }

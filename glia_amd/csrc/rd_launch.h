@@ -58,6 +58,15 @@ int launch_z_point(const LaunchCtx& c, int mode, int s_in, int s_out, int r_slot
 enum { ZUM_AXPBY = 0, ZUM_CGUPD = 1 };
 int launch_z_upd_r2c(const LaunchCtx& c, int mode, int ra, int rb, int rc, int rd, const double* sc, int s_out,
                      bool honor_done);
+// the elasticity passes fused over x-planes (plane_point.hip), on grids plane_supported takes:
+// F_yz(m F_yz^-1 in); where plane_io_supported, ZPM_SCREEN and ZPM_C2R_DOT with their Y pass
+// (plane_blocks(d) blocks of partials) and the two launch_z_upd_r2c modes with theirs
+bool plane_io_supported(const Dims& d);
+int plane_blocks(const Dims& d);
+int launch_plane_coef(const LaunchCtx& c, int s_in, int s_out, int r_slot, bool honor_done);
+int launch_plane_out(const LaunchCtx& c, int mode, int s_in, int r_out, int r_b, bool honor_done);
+int launch_plane_in(const LaunchCtx& c, int mode, int ra, int rb, int rc, int rd, const double* sc, int s_out,
+                    bool honor_done);
 // the elasticity CG's state machine in lane 0's PcgState (k_el_cg_begin / k_el_cg_fin)
 int launch_el_cg_begin(const LaunchCtx& c, double beta0, double dp0, double rnorm0, double ttol, double atol,
                        double dtol, int maxit);
@@ -94,8 +103,8 @@ int launch_lane_lin(const LaunchCtx& c, const int* nterms, const int (*lane)[4],
 // (honor_done: lanes whose CG has finished return at once)
 int launch_col_lin(const LaunchCtx& c, const int* nterms, const int (*lane)[4], const int (*slot)[4],
                    const int (*dir)[4], int s_out, bool honor_done);
-// out[q], q < nq: the Z-pass block partials (nq per block) of the c.nm lanes, summed on the device
-int launch_lane_part_sum(const LaunchCtx& c, int nq, double* out);
+// out[q], q < nq: the block partials (nq for each of nb blocks) of the c.nm lanes, summed on the device
+int launch_lane_part_sum(const LaunchCtx& c, int nb, int nq, double* out);
 // the elasticity preconditioner with F_d and U_d in lane d (members 0..2)
 int launch_el_prec_lanes(const LaunchCtx& c, int sf, int su, double mu, double lam, double scr, bool honor_done);
 int launch_bricks(const LaunchCtx& c, const BrickJob* jobs_host, int njobs, const double* taps_host, int tap_stride,

@@ -72,3 +72,54 @@ def test_zero_coefficient_and_a_field_written_after_creation():
     ref = apply_d(k.astype(np.float64), f.astype(np.float64))
     assert np.linalg.norm(s.get_field(0, "ct") - ref) < 5e-6 * np.linalg.norm(ref)
     s.close()
+
+
+def elastic(mu, lam, scr, avg):
+    n = mu.shape
+    w = [np.fft.fftfreq(n[0], 1.0 / n[0]), np.fft.fftfreq(n[1], 1.0 / n[1]), np.fft.rfftfreq(n[2], 1.0 / n[2])]
+    for a, m in zip(w, n):
+        a[np.abs(a) == m // 2] = 0.0
+    w = [w[0][:, None, None], w[1][None, :, None], w[2][None, None, :]]
+    r2c, c2r = np.fft.rfftn, lambda F: np.fft.irfftn(F, s=n, axes=(0, 1, 2))
+    w2 = sum(a * a for a in w)
+
+    def A(u):
+        U = [r2c(c) for c in u]
+        L = r2c(lam * c2r(1j * sum(a * F for a, F in zip(w, U))))
+        S = [[r2c(mu * c2r(1j * (w[j] * U[i] + w[i] * U[j]))) for j in range(3)] for i in range(3)]
+        return np.stack([c2r(1j * (sum(w[j] * S[i][j] for j in range(3)) + w[i] * L)) - scr * u[i] for i in range(3)])
+
+    def B(f):
+        F = [r2c(c) for c in f]
+        s1, s2 = -avg[2] - avg[0] * w2, avg[0] + avg[1]
+        c = s2 / (1.0 - w2 * s2 / s1) / s1 ** 2
+        wf = sum(a * G for a, G in zip(w, F))
+        return np.stack([c2r(F[d] / s1 + c * w[d] * wf) for d in range(3)])
+
+    return A, B
+
+
+@pytest.mark.parametrize("n", [(32, 32, 32), (32, 48, 64), (32, 80, 160), (32, 96, 96), (32, 128, 128), (32, 160, 160),
+                               (32, 192, 160), (32, 256, 256)])
+def test_elasticity_on_planes(n):
+    """Operator, preconditioner and a solve whose residual is measured with the FP64 operator; sizes with
+    whole and split planes, lines that do not fill a wave, and one whose one-way transforms stay separate."""
+    from glia_amd import elasticity
+    from glia_amd.synth import tissue_and_tumor
+    print("case plane elasticity", n, flush=True)
+    c, wm, gm, csf, vt, bg = tissue_and_tumor(n)
+    s = elasticity.ElasticitySolver(n)
+    s.set_material(c, wm, gm, csf, vt, bg)
+    mu, lam, scr, avg = s.material()
+    A, B = elastic(*[a.astype(np.float64) for a in (mu, lam, scr)], avg)
+    rng = np.random.default_rng(sum(n))
+    u = rng.standard_normal((3,) + n).astype(np.float32)
+    for got, ref in ((s.apply(u), A(u.astype(np.float64))), (s.precondition(u), B(u.astype(np.float64)))):
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert err < 5e-6, err  # as the diffusion operator's bound
+    f = (-1e2 * np.stack(np.gradient(c, *[2 * np.pi / m for m in n]))).astype(np.float32)
+    x, its, reason, _ = s.solve(f)
+    f = f.astype(np.float64)
+    res = np.linalg.norm(B(f - A(x.astype(np.float64)))) / np.linalg.norm(B(f))
+    assert reason == "rtol" and res < 1.01e-3, (its, reason, res)
+    s.close()
