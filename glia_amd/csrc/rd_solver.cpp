@@ -1930,12 +1930,13 @@ int RDEnsemble::smooth_field(int m, int rslot, double sigma) {
   const int* kr = smooth_kr_;
   const int stride = smooth_stride_;
   float* f = mh_[m].r[rslot];
-  float* scratch = reinterpret_cast<float*>(mh_[m].c[CS_T7]);  // n0*n1*n2 floats
+  // transform work slots of n0*n1*n2 floats each: the third pass ends in the field itself
+  float* s0 = reinterpret_cast<float*>(mh_[m].c[CS_T7]);
+  float* s1 = reinterpret_cast<float*>(mh_[m].c[CS_T6]);
   LaunchCtx c = ctx();
-  if (!rc) rc = launch_smooth_axis(c, f, scratch, 0, td, kr[0]);
-  if (!rc) rc = launch_smooth_axis(c, scratch, f, 1, td + stride, kr[1]);
-  if (!rc) rc = launch_smooth_axis(c, f, scratch, 2, td + 2 * stride, kr[2]);
-  if (!rc) rc = check(hipMemcpyAsync(f, scratch, sizeof(float) * d_.ng, hipMemcpyDeviceToDevice, stream_), "smooth copy");
+  if (!rc) rc = launch_smooth_axis(c, f, s0, 0, td, kr[0]);
+  if (!rc) rc = launch_smooth_axis(c, s0, s1, 1, td + stride, kr[1]);
+  if (!rc) rc = launch_smooth_axis(c, s1, f, 2, td + 2 * stride, kr[2]);
   return rc;
 }
 
