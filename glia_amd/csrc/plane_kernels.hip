@@ -35,6 +35,19 @@ __global__ void __launch_bounds__(256) k_plane_mask(const MemberDev* __restrict_
   if (threadIdx.x == 0) M.kmask[blockIdx.x] = mask;
 }
 
+// the planes with a nonzero as one bit each, for the X passes around the plane pass
+__global__ void __launch_bounds__(64) k_plane_bits(const MemberDev* __restrict__ mem, Dims d) {
+  const MemberDev& M = mem[blockIdx.x];
+  for (int i = 0; i < 4; i++) {
+    const int x = 64 * i + (int)threadIdx.x;
+    const unsigned long long b = __ballot(x < d.n0 && M.kmask[x] != 0);
+    if (threadIdx.x == 0) {
+      M.planes[2 * i] = (unsigned)b;
+      M.planes[2 * i + 1] = (unsigned)(b >> 32);
+    }
+  }
+}
+
 // Middle of the matvec on one plane and component: h = k * grad_d p on the grid, transformed back
 // along z and y.  From U and V (inverse X pass of p and of i w_x p):
 //   component x: out = F_yz(k F_yz^-1 V)                 y: out = i w_y F_yz(k F_yz^-1 (i w_y U))
@@ -44,7 +57,8 @@ __global__ void __launch_bounds__(256) k_plane_mask(const MemberDev* __restrict_
 template <int N1, int N2>
 __global__ void __launch_bounds__((PL<N1, N2>::TB), (PL<N1, N2>::MINW))
 k_plane_diff(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ tw1, const float2* __restrict__ twm,
-             const float2* __restrict__ tw2, int s_u, int s_v, int s_x, int s_y, int s_z, int k_slot) {
+             const float2* __restrict__ tw2, int s_u, int s_v, int s_x, int s_y, int s_z, int k_slot,
+             int use_planes) {
   using K = PL<N1, N2>;
   using RP = RealPart<K>;
   const MemberDev& Mb = mem[blockIdx.y];
@@ -66,7 +80,7 @@ k_plane_diff(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict
   // nothing to transform (the block's other plane, if any, included: with one plane to do, the other's
   // rows read as zero below and give zeros)
   if (mask == 0 && (K::CH == 1 || Mb.kmask[plane ^ 1] == 0)) {
-    if (L.y_on) {
+    if (L.y_on && !use_planes) {  // otherwise the X pass does not read these rows
 #pragma unroll 4
       for (int j = 0; j < K::RY; j++) (out + 4 * j * K::M)[(unsigned)(L.yt * K::M + L.yc)] = make_float2(0.0f, 0.0f);
     }
@@ -143,7 +157,7 @@ template <int N1, int N2>
 struct RunPlaneDiff {
   static int run(const LaunchCtx& c, int s_u, int s_v, int s_x, int s_y, int s_z, int k_slot) {
     k_plane_diff<N1, N2><<<dim3(3 * c.d.n0 / PL<N1, N2>::CH, c.nm), PL<N1, N2>::TB, 0, c.stream>>>(c.mem, c.d, c.tw1, c.twm, c.tw2, s_u, s_v,
-                                                                              s_x, s_y, s_z, k_slot);
+                                                                              s_x, s_y, s_z, k_slot, c.use_planes);
     return (int)hipGetLastError();
   }
 };
@@ -152,6 +166,7 @@ int launch_plane_diff(const LaunchCtx& c, int s_u, int s_v, int s_x, int s_y, in
 }
 int launch_plane_mask(const LaunchCtx& c, int k_slot, bool begin, double tau) {
   k_plane_mask<<<dim3(c.d.n0, c.nm), 256, 0, c.stream>>>(c.mem, c.d, k_slot, begin ? 1 : 0, tau);
+  if (c.use_planes) k_plane_bits<<<c.nm, 64, 0, c.stream>>>(c.mem, c.d);
   return (int)hipGetLastError();
 }
 

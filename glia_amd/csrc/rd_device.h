@@ -94,6 +94,7 @@ struct MemberDev {
   float* r[RS_NUM];
   PcgState* st;
   unsigned* kmask;     // per x-plane: its 32-line groups with a nonzero diffusion coefficient
+  unsigned* planes;    // the x-planes with a nonzero diffusion coefficient, one bit each (256 bits)
   double* part;        // per-workgroup partial sums (FP64)
   float2** hist;       // spectral states kept for the adjoint (store-all or checkpoints)
   float** chalf;       // real half-step states (adjoint_store), may be null

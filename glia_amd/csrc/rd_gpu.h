@@ -163,6 +163,23 @@ __device__ __forceinline__ void pcg_begin_state(PcgState* s, double tau) {
   }
 }
 
+// The x-planes on which the matvec's middle is not zero (MemberDev::planes), for the X passes around it:
+// the inverse pass need not write, nor the forward pass read, the other planes' rows.  A quarter of a
+// scan's planes hold no brain.  Without use every plane counts.
+struct PlaneBits {
+  unsigned w[9];
+  __device__ __forceinline__ PlaneBits(const MemberDev& M, int use) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) w[i] = use ? M.planes[i] : ~0u;
+    w[8] = ~0u;
+  }
+  // plane c + v with c known at compile time and v < 32
+  __device__ __forceinline__ bool on(int c, int v) const {
+    const uint64_t b = ((uint64_t)w[(c >> 5) + 1] << 32) | w[c >> 5];
+    return (b >> ((c & 31) + v)) & 1;
+  }
+};
+
 // the vector update of an elasticity CG iteration, from its state and, for the x and r update, the
 // summed <p, A p>: p = z + t p with t = beta / betaold (upd false: p = z, the first iteration and a
 // zero beta), or x += t p, r -= t w with t = beta / <p, A p> (upd false: none, where the CG stops on

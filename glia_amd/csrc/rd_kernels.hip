@@ -222,12 +222,14 @@ k_col_lin(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ 
 // first updated in place: p = B r (i == 0) or p = B r + (beta/betaold) p.
 template <int L, bool PUPD>
 __global__ void __launch_bounds__(CK<L>::TPB, CK<L>::VPT <= 16 ? GLIA_XI_MINW : 2)
-k_xi_grad(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ tw, int s_in, int s_r, int s_u, int s_v) {
+k_xi_grad(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ tw, int s_in, int s_r, int s_u, int s_v,
+          int use_planes) {
   constexpr int H = GLIA_NT_XI;
   const MemberDev& M = mem[blockIdx.y];
   const PcgState* st = M.st;
   if (st->done) return;
   GLIA_COL_PRELUDE(L)
+  const PlaneBits planes(M, use_planes);
   const Tile tl = col_tile(0, d);
   const float wy = wnum(tl.o, d.n1), wz = (float)(tl.c0 + col);
   GPtrT<H> pin = cptr<H>(M, s_in) + tl.base;
@@ -278,7 +280,7 @@ k_xi_grad(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ 
   fft2s<R1, R2, NT, +1>(b, exc, t, twl);
 #pragma unroll
   for (int j = 0; j < K::VOUT; j++) {
-    if (!K::out_ok(t, j)) continue;
+    if (!K::out_ok(t, j) || !planes.on(R1 * (j % R2) + (j / R2) * NT, t)) continue;
     const unsigned g = (unsigned)out_row<R1, R2, NT>(t, j) * tl.rs + col;
     U[g] = a[j];
     V[g] = b[j];
@@ -399,7 +401,7 @@ enum { XF_MATVEC = 0, XF_SETUP = 1, XF_D = 2 };
 template <int L, int MODE, bool SUM>
 __global__ void __launch_bounds__(CK<L>::TPB, CK<L>::VPT <= 16 ? GLIA_XF_MINW : 2)
 k_xf_div(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ tw, int s_yx, int s_rr, int s_rb, int s_p,
-         int s_out) {
+         int s_out, int use_planes) {
   constexpr int H = GLIA_NT_XF;
   const MemberDev& M = mem[blockIdx.y];
   const PcgState* st = M.st;
@@ -416,16 +418,34 @@ k_xf_div(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ t
   const double wgt = (tl.c0 + col == 0) ? 1.0 : 2.0;
   constexpr bool PF = K::VPT <= GLIA_XF_PF_VPT && GLIA_XF_PF;
   float2 a[K::VPT], b[K::VPT], pv[PF ? K::VPT : 1];
-#pragma unroll
-  for (int j = 0; j < K::VIN; j++) {
-    const unsigned g = (unsigned)in_row<R1, R2, NT>(t, j) * tl.rs + col;
-    a[j] = Yx[g];
-    b[j] = Rr[g];
-  }
   if constexpr (SUM) {
+    // a skipped plane's row reads row 0 instead (one cached line) and counts as zero
+    const PlaneBits planes(M, use_planes);
     GPtrT<H> Rb = cptr<H>(M, s_rb) + tl.base;
+    auto on = [&](int j) { return planes.on(R2 * (j % R1) + (j / R1) * NT, t); };
 #pragma unroll
-    for (int j = 0; j < K::VIN; j++) b[j] = cadd(b[j], Rb[(unsigned)in_row<R1, R2, NT>(t, j) * tl.rs + col]);
+    for (int j = 0; j < K::VIN; j++) {
+      const unsigned g = (on(j) ? (unsigned)in_row<R1, R2, NT>(t, j) * tl.rs : 0u) + col;
+      a[j] = Yx[g];
+      b[j] = Rr[g];
+    }
+#pragma unroll
+    for (int j = 0; j < K::VIN; j++) {
+      const unsigned g = (on(j) ? (unsigned)in_row<R1, R2, NT>(t, j) * tl.rs : 0u) + col;
+      b[j] = cadd(b[j], Rb[g]);
+    }
+#pragma unroll
+    for (int j = 0; j < K::VIN; j++) {
+      a[j] = make_float2(on(j) ? a[j].x : 0.0f, on(j) ? a[j].y : 0.0f);
+      b[j] = make_float2(on(j) ? b[j].x : 0.0f, on(j) ? b[j].y : 0.0f);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < K::VIN; j++) {
+      const unsigned g = (unsigned)in_row<R1, R2, NT>(t, j) * tl.rs + col;
+      a[j] = Yx[g];
+      b[j] = Rr[g];
+    }
   }
   // the operand of the output stage is loaded before the transforms (a barrier would otherwise
   // keep its loads behind them)
@@ -2081,9 +2101,9 @@ struct RunXiGrad {
   static int run(const LaunchCtx& c, int s_in, int s_r, int s_u, int s_v, bool pupd) {
     dim3 g(c.d.n1 * (c.d.m2 / 16), c.nm);
     if (pupd)
-      k_xi_grad<L, true><<<g, CK<L>::TPB, 0, c.stream>>>(c.mem, c.d, c.tw0, s_in, s_r, s_u, s_v);
+      k_xi_grad<L, true><<<g, CK<L>::TPB, 0, c.stream>>>(c.mem, c.d, c.tw0, s_in, s_r, s_u, s_v, c.use_planes);
     else
-      k_xi_grad<L, false><<<g, CK<L>::TPB, 0, c.stream>>>(c.mem, c.d, c.tw0, s_in, s_r, s_u, s_v);
+      k_xi_grad<L, false><<<g, CK<L>::TPB, 0, c.stream>>>(c.mem, c.d, c.tw0, s_in, s_r, s_u, s_v, c.use_planes);
     GLIA_CHECK_LAUNCH();
     return 0;
   }
@@ -2139,13 +2159,13 @@ struct RunXfDiv {
     const dim3 g(c.d.n1 * (c.d.m2 / 16), c.nm);
     constexpr int tb = CK<L>::TPB;
     if (s_rb >= 0)
-      k_xf_div<L, MODE, true><<<g, tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_rb, s_p, s_out);
+      k_xf_div<L, MODE, true><<<g, tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_rb, s_p, s_out, c.use_planes);
     else if (c.xf_split == 2)
       k_xf_div_s3<L, MODE><<<g, 3 * tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
     else if (c.xf_split)
       k_xf_div_s<L, MODE><<<g, 2 * tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, s_p, s_out);
     else
-      k_xf_div<L, MODE, false><<<g, tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, 0, s_p, s_out);
+      k_xf_div<L, MODE, false><<<g, tb, 0, c.stream>>>(c.mem, c.d, c.tw0, s_yx, s_rr, 0, s_p, s_out, 0);
     GLIA_CHECK_LAUNCH();
     return 0;
   }

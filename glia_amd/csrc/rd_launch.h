@@ -19,6 +19,9 @@ struct LaunchCtx {
   // variant of the forward divergence passes: split-group kernels (one field per thread group)
   // instead of one group holding every field; chosen per handle (autotuned or by default)
   int yf_split = 0, xf_split = 0;
+  // the matvec's X passes and plane pass leave out the planes where k is zero (launch_plane_mask with
+  // the same setting first)
+  int use_planes = 0;
 };
 
 // modes of launch_xf_div and launch_z_point (values match the kernel enums)

@@ -88,6 +88,14 @@ LaunchCtx RDEnsemble::ctx() const {
   return c;
 }
 
+// the context of the matvec's passes.  From 2^21 points the X passes leave out the rows of planes where k
+// is zero; below, launches are what counts and the extra one per solve is saved.
+LaunchCtx RDEnsemble::matvec_ctx() const {
+  LaunchCtx c = ctx();
+  c.use_planes = plane_ && (int64_t)c.nm * d_.ng >= ((int64_t)1 << 21) ? 1 : 0;
+  return c;
+}
+
 // launch context of member m alone
 static LaunchCtx member_ctx(LaunchCtx c, const MemberDev* md, int m) {
   c.mem = md + m;
@@ -225,7 +233,8 @@ int RDEnsemble::alloc_member(int m) {
   nb = std::max<int64_t>(nb, (int64_t)ew_blocks() * 2);
   GLIA_HIP(hipMalloc(&part_[m], sizeof(double) * nb));
   M.part = part_[m];
-  GLIA_HIP(hipMalloc(&M.kmask, sizeof(unsigned) * d_.n0));
+  GLIA_HIP(hipMalloc(&M.kmask, sizeof(unsigned) * (d_.n0 + 8)));
+  M.planes = M.kmask + d_.n0;
   int rc = alloc_history(m);
   if (rc) return rc;
   M.kr_gm = (float)cfg_.k_gm_wm;
@@ -817,7 +826,7 @@ int RDEnsemble::set_spectrum(int m, int cslot, const float2* host) {
 // the passes of the matvec between its X passes, from U and V in CS_T0 and CS_T1: gradient, product
 // with the real slot k_slot, forward transforms along z and y
 int RDEnsemble::middle_passes(int k_slot, bool timed) {
-  LaunchCtx c = ctx();
+  LaunchCtx c = matvec_ctx();
   auto mark = [&](int kind, bool begin) {
     if (timed) prof_mark(kind, begin);
   };
@@ -841,19 +850,18 @@ int RDEnsemble::middle_passes(int k_slot, bool timed) {
 
 // the forward X pass after middle_passes
 int RDEnsemble::close_divergence(int mode, int s_p, int s_out) {
-  if (plane_) return launch_xf_div(ctx(), mode, CS_T2, CS_T3, CS_T4, s_p, s_out);
+  if (plane_) return launch_xf_div(matvec_ctx(), mode, CS_T2, CS_T3, CS_T4, s_p, s_out);
   return launch_xf_div(ctx(), mode, CS_T0, CS_T1, -1, s_p, s_out);
 }
 
 // the start of a CN solve with the diffusion coefficient RS_K
 int RDEnsemble::solve_begin(double tau) {
-  return plane_ ? launch_plane_mask(ctx(), RS_K, true, tau) : launch_pcg_begin(ctx(), tau);
+  return plane_ ? launch_plane_mask(matvec_ctx(), RS_K, true, tau) : launch_pcg_begin(ctx(), tau);
 }
 
 // b - A x0 for x0 = c: r = tau D c, with the partial norms of B b and B r (KSPConvergedDefault)
 int RDEnsemble::matvec_setup(int sx) {
-  LaunchCtx c = ctx();
-  GLIA_TRYC(launch_xi_grad(c, sx, 0, CS_T0, CS_T1, false));
+  GLIA_TRYC(launch_xi_grad(matvec_ctx(), sx, 0, CS_T0, CS_T1, false));
   GLIA_TRYC(middle_passes(RS_K));
   GLIA_TRYC(close_divergence(XFM_SETUP, sx, CS_R));
   return 0;
@@ -1141,7 +1149,7 @@ int RDEnsemble::launch_iteration(int sx, int slot) {
   LaunchCtx c = ctx();
   const int nbx = xf_div_blocks(d_);
   prof_mark(PK_XI_PUPD, true);
-  GLIA_TRYC(launch_xi_grad(c, CS_P, CS_R, CS_T0, CS_T1, true));
+  GLIA_TRYC(launch_xi_grad(matvec_ctx(), CS_P, CS_R, CS_T0, CS_T1, true));
   prof_mark(PK_XI_PUPD, false);
   int rc = middle_passes(RS_K, true);
   if (rc) return rc;
@@ -1366,9 +1374,8 @@ int RDEnsemble::tangent_step(int sx, int cslot_c) {
 int RDEnsemble::apply_dsec(int in, int out) {
   int rc = clear_done();
   if (rc) return rc;
-  LaunchCtx c = ctx();
-  if (plane_) GLIA_TRYC(launch_plane_mask(c, RS_KS, false, 0.0));
-  GLIA_TRYC(launch_xi_grad(c, in, 0, CS_T0, CS_T1, false));
+  if (plane_) GLIA_TRYC(launch_plane_mask(matvec_ctx(), RS_KS, false, 0.0));
+  GLIA_TRYC(launch_xi_grad(matvec_ctx(), in, 0, CS_T0, CS_T1, false));
   GLIA_TRYC(middle_passes(RS_KS));
   GLIA_TRYC(close_divergence(XFM_D, in, out));
   return 0;
@@ -1754,9 +1761,8 @@ int RDEnsemble::apply_d_field(int rin, int rout) {
   if (rc) return rc;
   rc = clear_done();
   if (rc) return rc;
-  LaunchCtx c = ctx();
-  if (plane_) GLIA_TRYC(launch_plane_mask(c, RS_K, false, 0.0));
-  GLIA_TRYC(launch_xi_grad(c, CS_X, 0, CS_T0, CS_T1, false));
+  if (plane_) GLIA_TRYC(launch_plane_mask(matvec_ctx(), RS_K, false, 0.0));
+  GLIA_TRYC(launch_xi_grad(matvec_ctx(), CS_X, 0, CS_T0, CS_T1, false));
   GLIA_TRYC(middle_passes(RS_K));
   GLIA_TRYC(close_divergence(XFM_D, CS_X, CS_T5));
   rc = inverse_to_real(CS_T5, CS_T6, rout);

@@ -220,6 +220,7 @@ class RDEnsemble {
   int copy_sync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind);
   int fail(int code, const std::string& msg);
   LaunchCtx ctx() const;
+  LaunchCtx matvec_ctx() const;
 
   void smoother_taps(double sigma, std::vector<double>& taps, int kr[3], int& stride) const;
   int smooth_taps_for(double sigma);
