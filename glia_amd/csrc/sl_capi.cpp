@@ -84,10 +84,14 @@ int trajectories(glia_sl_s* h, double dt) {
   return 0;
 }
 
+// one launch over F's fields; a launch with a mass-conserving field on new trajectories (or a new
+// velocity) interpolates div v at the departure points along the way
 int apply(glia_sl_s* h, const SLFields& F, double dt) {
+  const bool fresh = F.any_mass && !h->div_ok;
   const int rc = glia::sl::launch_sl_apply(h->d, h->st, F, h->q[0], h->q[1], h->q[2],
-                                           h->e->field_ptr(0, glia::RS_VT), h->dvi, (float)dt);
+                                           h->e->field_ptr(0, glia::RS_VT), h->dvi, fresh, (float)dt);
   if (rc) return hip_fail(h, (hipError_t)rc, "advection launch");
+  if (fresh) h->div_ok = true;
   return 0;
 }
 
@@ -101,14 +105,11 @@ SLFields one_field(const float* in, float* out, int mode) {
   return F;
 }
 
-// div v on the grid (spectral, computeDivergence) and at the departure points
+// div v on the grid (spectral, computeDivergence) for the next apply, when it has not been used yet
 int ensure_div(glia_sl_s* h) {
   if (h->div_ok) return 0;
-  int rc = h->e->divergence(glia::RS_WM, glia::RS_GM, glia::RS_CSF, glia::RS_VT);
-  if (rc) return fail(h, rc, h->e->error());
-  if ((rc = apply(h, one_field(h->e->field_ptr(0, glia::RS_VT), h->dvi, GLIA_SL_PURE_ADVECTION), 0.0))) return rc;
-  h->div_ok = true;
-  return 0;
+  const int rc = h->e->divergence(glia::RS_WM, glia::RS_GM, glia::RS_CSF, glia::RS_VT);
+  return rc ? fail(h, rc, h->e->error()) : 0;
 }
 
 bool valid_kind(int kind) { return kind == GLIA_RD_HOST || kind == GLIA_RD_DEVICE; }

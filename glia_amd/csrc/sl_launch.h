@@ -25,7 +25,7 @@ struct SLFields {
 int launch_sl_trajectories(const SLDims& d, hipStream_t st, const float* vx, const float* vy, const float* vz,
                            float sx, float sy, float sz, float* qx, float* qy, float* qz);
 int launch_sl_apply(const SLDims& d, hipStream_t st, const SLFields& F, const float* qx, const float* qy,
-                    const float* qz, const float* dv, const float* dvi, float dt);
+                    const float* qz, const float* dv, float* dvi, bool new_dvi, float dt);
 
 }  // namespace sl
 }  // namespace glia
