@@ -314,8 +314,9 @@ int glia_rd_use_graphs(glia_rd_t h, int enable);
    its Y and Z passes fused and these variants are not on its path. */
 int glia_rd_autotune(glia_rd_t h, const char* cache_path, int* choice);
 /* Time steps replayed from captured graphs (glia_rd_use_graphs on, store-all history): each
-   forward and adjoint step runs as one graph whose CG loops are unrolled to the last iteration
-   counts plus one, and the host reads each solve's end-of-solve flag once per step.  A step
+   forward and adjoint step runs as one graph whose CG loops are unrolled to the counts of the
+   same step in the last evaluation plus one (first evaluation: the previous step's, and eager steps
+   from 2^22 points times members), and the host reads each solve's end-of-solve flag once per step.  A step
    whose solve needed more iterations runs again eagerly from its stored start.  launched and
    reruns count such steps since creation, cached the graphs held. */
 int glia_rd_step_info(glia_rd_t h, long long* launched, long long* reruns, int* cached);
