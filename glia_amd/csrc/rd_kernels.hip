@@ -1661,7 +1661,33 @@ __global__ void __launch_bounds__(256) k_support_count(const float* __restrict__
   cnt[t] = num;
 }
 
-// The same with the tap radius known at compile time, OUT consecutive points of the axis per thread: a
+// the same with the tap radius known at compile time, so that every load of a point is issued before its
+// sum (the same bits): for axes too short for the kernels below and z lines longer than 1024 points
+template <int KR>
+__global__ void __launch_bounds__(256) k_smooth_point(const float* __restrict__ in, float* __restrict__ out, Dims d,
+                                                      int axis, const double* __restrict__ taps) {
+  const int z = (int)(blockIdx.x * 64 + threadIdx.x), y = (int)(blockIdx.y * 4 + threadIdx.y), x = (int)blockIdx.z;
+  if (z >= d.n2 || y >= d.n1) return;
+  const int n = axis == 0 ? d.n0 : (axis == 1 ? d.n1 : d.n2);
+  const unsigned st = axis == 0 ? (unsigned)(d.n1 * d.n2) : (axis == 1 ? (unsigned)d.n2 : 1u);
+  const int ca = axis == 0 ? x : (axis == 1 ? y : z);
+  const unsigned i = ((unsigned)x * (unsigned)d.n1 + (unsigned)y) * (unsigned)d.n2 + (unsigned)z;
+  const unsigned base = i - (unsigned)ca * st;
+  float v[2 * KR + 1];
+#pragma unroll
+  for (int s = -KR; s <= KR; s++) {
+    int q = ca - s;
+    q += (q < 0) ? n : 0;
+    q -= (q >= n) ? n : 0;
+    v[s + KR] = in[base + (unsigned)q * st];
+  }
+  double acc = 0.0;
+#pragma unroll
+  for (int s = -KR; s <= KR; s++) acc += taps[s + KR] * (double)v[s + KR];
+  out[i] = (float)acc;
+}
+
+// The same again with OUT consecutive points of the axis per thread (the last group may be short): a
 // value is loaded and widened once for the OUT sums it enters.  Every sum runs in k_smooth_axis's order
 // (the input index falls), so the results are the same bit for bit.  Axes 0 and 1: lanes along z.
 // One point a thread spent its time on 2 KR + 1 loads through L1 (192^3, KR = 12: 61 us a pass); with
@@ -1697,17 +1723,20 @@ __global__ void __launch_bounds__(256) k_smooth_xy(const float* __restrict__ in,
     }
   }
 #pragma unroll
-  for (int o = 0; o < OUT; o++) out[base + (unsigned)(c0 + o) * st] = (float)acc[o];
+  for (int o = 0; o < OUT; o++)
+    if (c0 + o < n) out[base + (unsigned)(c0 + o) * st] = (float)acc[o];
 }
 
 // axis 2: four consecutive points per thread, lines with their periodic ends in LDS, read in 16-byte words
-// (192^3, KR = 12: 61 -> 25 us)
+// (192^3, KR = 12: 61 -> 25 us).  vec: the outputs are stored in 16-byte words, else one by one (lengths
+// that are no multiple of 4, fields off the 16-byte grid).
 template <int KR>
 __global__ void __launch_bounds__(256) k_smooth_z(const float* __restrict__ in, float* __restrict__ out, Dims d, int rows,
-                                                  const double* __restrict__ taps) {
+                                                  int vec, const double* __restrict__ taps) {
   constexpr int PAD = (4 - KR % 4) % 4, WIN = (PAD + 2 * KR + 4 + 3) / 4 * 4;  // window of a thread, whole words
   extern __shared__ __align__(16) float line[];
-  const int pitch = d.n2 + WIN;  // entry e of a line holds z = e - KR - PAD
+  const int per = (d.n2 + 3) / 4;   // threads of a line
+  const int pitch = 4 * per + WIN;  // entry e of a line holds z = e - KR - PAD
   const int64_t r0 = (int64_t)blockIdx.x * rows;
   const int64_t nrows = (int64_t)d.n0 * d.n1;
   for (int e = threadIdx.x; e < rows * pitch; e += 256) {
@@ -1718,7 +1747,7 @@ __global__ void __launch_bounds__(256) k_smooth_z(const float* __restrict__ in, 
     if (r0 + r < nrows) line[e] = in[(unsigned)((r0 + r) * d.n2 + z)];
   }
   __syncthreads();
-  const int per = d.n2 / 4, r = (int)threadIdx.x / per, z0 = 4 * ((int)threadIdx.x - r * per);
+  const int r = (int)threadIdx.x / per, z0 = 4 * ((int)threadIdx.x - r * per);
   if (r >= rows || r0 + r >= nrows) return;
   float v[WIN];
 #pragma unroll
@@ -1733,8 +1762,14 @@ __global__ void __launch_bounds__(256) k_smooth_z(const float* __restrict__ in, 
       if (s >= -KR && s <= KR) acc[o] += taps[s + KR] * x;
     }
   }
-  float4 w = make_float4((float)acc[0], (float)acc[1], (float)acc[2], (float)acc[3]);
-  *reinterpret_cast<float4*>(out + (unsigned)((r0 + r) * d.n2 + z0)) = w;
+  float* w = out + (unsigned)((r0 + r) * d.n2 + z0);
+  if (vec) {
+    *reinterpret_cast<float4*>(w) = make_float4((float)acc[0], (float)acc[1], (float)acc[2], (float)acc[3]);
+  } else {
+#pragma unroll
+    for (int o = 0; o < 4; o++)
+      if (z0 + o < d.n2) w[o] = (float)acc[o];
+  }
 }
 
 // one axis of the separable smoothing: the kept extent shrinks by 2*kr[axis] along 'axis'; the
@@ -2343,24 +2378,34 @@ int launch_support_count(const LaunchCtx& c, const float* f, int step, int l0, i
   return 0;
 }
 
+// The kernels that share loads between points index a window of up to KR + 10 points past either end of an
+// axis and wrap it once; shorter axes, z lines that a block's threads do not cover and offsets beyond 32
+// bits take one point a thread.  182 x 218 x 182 with KR = 12, all three passes: 83 us, against 226 with one
+// point a thread on every axis and 415 in the loop of unknown radius.
 template <int KR>
 static void smooth_launch(const LaunchCtx& c, const float* in, float* out, int axis, const double* taps) {
   const Dims& d = c.d;
+  const dim3 b(64, 4);
+  const int n = axis == 0 ? d.n0 : (axis == 1 ? d.n1 : d.n2);
+  const unsigned gx = (unsigned)((d.n2 + 63) / 64), gy = (unsigned)((d.n1 + 3) / 4);
+  if (n < KR + 16 || d.ng >= (int64_t)1 << 31 || (axis == 2 && n > 1024)) {
+    k_smooth_point<KR><<<dim3(gx, gy, (unsigned)d.n0), b, 0, c.stream>>>(in, out, d, axis, taps);
+    return;
+  }
   if (axis == 2) {
-    const int rows = 1024 / d.n2;  // 256 threads of four points
+    const int per = (n + 3) / 4, rows = 256 / per;  // 256 threads of four points
     const int64_t nrows = (int64_t)d.n0 * d.n1;
+    const int vec = n % 4 == 0 && (uintptr_t)out % 16 == 0 ? 1 : 0;
     constexpr int PAD = (4 - KR % 4) % 4, WIN = (PAD + 2 * KR + 4 + 3) / 4 * 4;
-    k_smooth_z<KR><<<(unsigned)((nrows + rows - 1) / rows), 256, sizeof(float) * rows * (d.n2 + WIN), c.stream>>>(
-        in, out, d, rows, taps);
+    k_smooth_z<KR><<<(unsigned)((nrows + rows - 1) / rows), 256, sizeof(float) * rows * (4 * per + WIN), c.stream>>>(
+        in, out, d, rows, vec, taps);
     return;
   }
   // eight points a thread where that leaves 2048 waves (2^20 points); two below
   const auto go = [&](auto outs) {
     constexpr int OUT = decltype(outs)::value;
-    const dim3 b(64, 4);
-    const unsigned gx = (unsigned)((d.n2 + 63) / 64);
-    const dim3 g = axis == 0 ? dim3(gx, (unsigned)((d.n1 + 3) / 4), (unsigned)(d.n0 / OUT))
-                             : dim3(gx, (unsigned)((d.n1 / OUT + 3) / 4), (unsigned)d.n0);
+    const unsigned groups = (unsigned)((n + OUT - 1) / OUT);
+    const dim3 g = axis == 0 ? dim3(gx, gy, groups) : dim3(gx, (groups + 3) / 4, (unsigned)d.n0);
     k_smooth_xy<KR, OUT><<<g, b, 0, c.stream>>>(in, out, d, axis, taps);
   };
   if (d.ng >= (int64_t)1 << 20)
@@ -2371,13 +2416,9 @@ static void smooth_launch(const LaunchCtx& c, const float* in, float* out, int a
 
 int launch_smooth_axis(const LaunchCtx& c, const float* in, float* out, int axis, const double* taps, int kr) {
   const dim3 g((unsigned)((c.d.n2 + 63) / 64), (unsigned)((c.d.n1 + 3) / 4), (unsigned)c.d.n0), b(64, 4);
-  // the kernels with a known radius take the lengths the engine plans: multiples of 16, z lines of at
-  // most 1024 points, radii below half the axis, fields in 16-byte words
-  const bool planned = c.d.n0 % 16 == 0 && c.d.n1 % 16 == 0 && c.d.n2 % 16 == 0 && c.d.n2 <= 1024 &&
-                       ((uintptr_t)in | (uintptr_t)out) % 16 == 0 && c.d.ng < ((int64_t)1 << 31);
 #define GLIA_SMK(K) \
   case K: smooth_launch<K>(c, in, out, axis, taps); break;
-  switch (planned ? kr : 0) {
+  switch (kr) {
     GLIA_SMK(1) GLIA_SMK(2) GLIA_SMK(3) GLIA_SMK(4) GLIA_SMK(5) GLIA_SMK(6) GLIA_SMK(7) GLIA_SMK(8)
     GLIA_SMK(9) GLIA_SMK(10) GLIA_SMK(11) GLIA_SMK(12) GLIA_SMK(13) GLIA_SMK(14) GLIA_SMK(15) GLIA_SMK(16)
     default: k_smooth_axis<<<g, b, 0, c.stream>>>(in, out, c.d, axis, taps, kr); break;
