@@ -166,17 +166,28 @@ __device__ __forceinline__ void pcg_begin_state(PcgState* s, double tau) {
 // The x-planes on which the matvec's middle is not zero (MemberDev::planes), for the X passes around it:
 // the inverse pass need not write, nor the forward pass read, the other planes' rows.  A quarter of a
 // scan's planes hold no brain.  Without use every plane counts.
+// The words are named one by one: an array of them stayed in scratch memory (16-40 bytes a lane, 11
+// spilled registers in the 256-point inverse pass), which cost more traffic than the skipped rows saved:
+// inverse and forward X pass 122 and 121 -> 106 and 112 us at 8 x 160^3, 234 and 259 -> 203 and 220 at 4 x 256^3
+// (115 and 127, 237 and 257 with every row written and read).
 struct PlaneBits {
-  unsigned w[9];
+  uint64_t q0, q1, q2, q3;
   __device__ __forceinline__ PlaneBits(const MemberDev& M, int use) {
-#pragma unroll
-    for (int i = 0; i < 8; i++) w[i] = use ? M.planes[i] : ~0u;
-    w[8] = ~0u;
+    const auto word = [&](int i) -> uint64_t {
+      return use ? (uint64_t)M.planes[2 * i + 1] << 32 | M.planes[2 * i] : ~0ull;
+    };
+    q0 = word(0), q1 = word(1), q2 = word(2), q3 = word(3);
   }
-  // plane c + v with c known at compile time and v < 32
+  __device__ __forceinline__ unsigned word32(int i) const {
+    const uint64_t q = i < 2 ? q0 : i < 4 ? q1 : i < 6 ? q2 : i < 8 ? q3 : ~0ull;
+    return (unsigned)(i & 1 ? q >> 32 : q);
+  }
+  // plane c + v with c known at compile time and v < NT <= 32
+  template <int NT>
   __device__ __forceinline__ bool on(int c, int v) const {
-    const uint64_t b = ((uint64_t)w[(c >> 5) + 1] << 32) | w[c >> 5];
-    return (b >> ((c & 31) + v)) & 1;
+    const int sh = c & 31;
+    if (sh + NT <= 32) return (word32(c >> 5) >> (sh + v)) & 1;
+    return ((((uint64_t)word32((c >> 5) + 1) << 32) | word32(c >> 5)) >> (sh + v)) & 1;
   }
 };
 

@@ -278,10 +278,14 @@ k_xi_grad(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ 
   fft2s<R1, R2, NT, +1>(a, exc, t, twl);
   __syncthreads();
   fft2s<R1, R2, NT, +1>(b, exc, t, twl);
+  // the lane's number renewed: the planes' bits and the rows' offsets are not made before the transforms
+  // and held through them (16 spilled registers at 256 points)
+  int to = t;
+  asm volatile("" : "+v"(to));
 #pragma unroll
   for (int j = 0; j < K::VOUT; j++) {
-    if (!K::out_ok(t, j) || !planes.on(R1 * (j % R2) + (j / R2) * NT, t)) continue;
-    const unsigned g = (unsigned)out_row<R1, R2, NT>(t, j) * tl.rs + col;
+    if (!K::out_ok(to, j) || !planes.on<NT>(R1 * (j % R2) + (j / R2) * NT, to)) continue;
+    const unsigned g = (unsigned)out_row<R1, R2, NT>(to, j) * tl.rs + col;
     U[g] = a[j];
     V[g] = b[j];
   }
@@ -422,7 +426,7 @@ k_xf_div(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__ t
     // a skipped plane's row reads row 0 instead (one cached line) and counts as zero
     const PlaneBits planes(M, use_planes);
     GPtrT<H> Rb = cptr<H>(M, s_rb) + tl.base;
-    auto on = [&](int j) { return planes.on(R2 * (j % R1) + (j / R1) * NT, t); };
+    auto on = [&](int j) { return planes.on<NT>(R2 * (j % R1) + (j / R1) * NT, t); };
 #pragma unroll
     for (int j = 0; j < K::VIN; j++) {
       const unsigned g = (on(j) ? (unsigned)in_row<R1, R2, NT>(t, j) * tl.rs : 0u) + col;

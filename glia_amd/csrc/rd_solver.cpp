@@ -89,7 +89,10 @@ LaunchCtx RDEnsemble::ctx() const {
 }
 
 // the context of the matvec's passes.  From 2^21 points the X passes leave out the rows of planes where k
-// is zero; below, launches are what counts and the extra one per solve is saved.
+// is zero; below, launches are what counts and the extra one per solve is saved.  An iteration's X and plane
+// passes with a scan's zero planes, left out against passed over: 8 x 128^3 184 against 196 us, 8 x 160^3 419
+// against 458, 4 x 192^3 366 against 399, 256^3 238 against 257; below 2^21 points (128 x 64 x 64, 96^3) and
+// with a coefficient that is zero nowhere within 1 us either way.
 LaunchCtx RDEnsemble::matvec_ctx() const {
   LaunchCtx c = ctx();
   c.use_planes = plane_ && (int64_t)c.nm * d_.ng >= ((int64_t)1 << 21) ? 1 : 0;

@@ -28,6 +28,8 @@ def fields(n, kind, rng):
         k[:, :, n[2] // 2:] = 0.0        # half of every line
         k[n[0] // 4 + 1] = 0.0
         k[n[0] // 4 + 1, n[1] // 3, 5] = 0.7  # one nonzero in a plane
+    if kind == "stripes":
+        k[rng.random(n[0]) < 0.5] = 0.0  # scattered zero planes, in every word of their mask
     return k.astype(np.float32)
 
 
@@ -51,6 +53,35 @@ def test_operator_on_planes(n, kind):
         err = np.linalg.norm(s.get_field(m, "ct") - ref) / np.linalg.norm(ref)
         # six transforms of log2(n) <= 24 levels in FP32: 24 eps = 1.4e-6 a transform at the worst
         assert err < 5e-6, err
+    s.close()
+
+
+@pytest.mark.parametrize("kind", ["stripes", "dense", "zero"])
+@pytest.mark.parametrize("n", [(48, 160, 160), (64, 160, 160), (64, 128, 128), (80, 128, 128), (96, 128, 96), (128, 96, 96),
+                               (160, 96, 96), (192, 64, 96), (256, 64, 64)])
+def test_operator_with_planes_left_out(n, kind):
+    """From 2^21 points the X passes leave out the rows of planes where k is zero: every X length, two planes
+    a block of which one is zero, and rows that hold another field's values from the call before."""
+    from glia_amd import rd
+    print("case planes left out", n, kind, flush=True)
+    assert 2 * n[0] * n[1] * n[2] >= 2 ** 21
+    rng = np.random.default_rng([n[0], n[1], n[2], len(kind)])
+    s = rd.RDSolver(n, nmembers=2)
+    f = [rng.standard_normal(n).astype(np.float32) for _ in range(2)]
+    k = [fields(n, kind, rng) if kind != "zero" else np.zeros(n, np.float32), fields(n, "stripes", rng)]
+    for m in range(2):  # leaves other values in every row of the work slots
+        s.set_field(m, "k", np.ones(n, np.float32))
+        s.set_field(m, "work", 1e3 * f[1 - m])
+    s.apply_d("work", "ct")
+    for m in range(2):
+        s.set_field(m, "k", k[m])
+        s.set_field(m, "work", f[m])
+    s.apply_d("work", "ct")
+    for m in range(2):
+        ref = apply_d(k[m].astype(np.float64), f[m].astype(np.float64))
+        err = np.linalg.norm(s.get_field(m, "ct") - ref)
+        # the bound of test_operator_on_planes; an operator that is zero gives exactly zero
+        assert err <= 5e-6 * np.linalg.norm(ref), err
     s.close()
 
 
