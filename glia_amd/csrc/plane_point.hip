@@ -102,15 +102,20 @@ k_plane_coef(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict
   y_store<K>(uniform(cptr<0>(Mb, s_out) + base), L, v);
 }
 
-// pairs a lane takes together: they divide its share of a part
+// Pairs a lane takes together: they divide its share of a part.  The last wave of 48 or 80 lines has half of
+// its lines, which are the first half of every lane's pairs: it takes half of the groups (skipping the lines
+// past the last one by one made every load a branch: 96 x 80 x 160, a CG iteration 447 -> 339 us).
 template <class K>
 struct PairGroup {
-  static constexpr int CNT = RealPart<K>::CNT;
-  static constexpr int value = CNT % 8 == 0 ? 8 : (CNT % 6 == 0 ? 6 : 5);
-  static_assert(CNT % value == 0, "a lane's pairs come in whole groups");
+  static constexpr int CNT = RealPart<K>::CNT, LAST = K::LINES % 32 ? CNT / 2 : CNT;
+  static constexpr int value = LAST % 8 == 0 ? 8 : (LAST % 6 == 0 ? 6 : (LAST % 5 == 0 ? 5 : 4));
+  static_assert(LAST % value == 0, "a lane's pairs come in whole groups");
+  static_assert(K::LINES % 32 == 0 || (K::LINES % 32 == 16 && CNT % 2 == 0 && RealPart<K>::PM % 4 == 0),
+                "half of the last wave's lines are half of every lane's pairs");
+  static __device__ __forceinline__ int count(int wave) { return wave == K::WZ - 1 ? LAST : CNT; }
 };
 // A group of the pairs of one part of the wave's lines in memory order: fn(i, offset in the plane, LDS
-// index of the pair), i < PairGroup, skipping lines past the plane's last.
+// index of the pair), i < PairGroup.
 template <class K, int PART, class Fn>
 __device__ __forceinline__ void line_pairs(int wave, int i0, Fn fn) {
   using RP = RealPart<K>;
@@ -118,8 +123,7 @@ __device__ __forceinline__ void line_pairs(int wave, int i0, Fn fn) {
 #pragma unroll
   for (int i = 0; i < PairGroup<K>::value; i++) {
     const int e = (i0 + i) * 64 + lane, row = wave * 32 + e / RP::PM, n = e % RP::PM;
-    if (K::LINES % 32 == 0 || row < K::LINES)
-      fn(i, (unsigned)(row * K::M + PART * RP::PM + n), K::SPLIT ? row * K::P + 2 * n : row * K::P + n);
+    fn(i, (unsigned)(row * K::M + PART * RP::PM + n), K::SPLIT ? row * K::P + 2 * n : row * K::P + n);
   }
 }
 template <class K>
@@ -198,7 +202,7 @@ k_plane_out(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict_
       wave_fence();
       constexpr int C = PairGroup<K>::value;
 #pragma unroll 1
-      for (int i0 = 0; i0 < RP::CNT; i0 += C) {
+      for (int i0 = 0; i0 < PairGroup<K>::count(B.wave); i0 += C) {
         float2 a[C], b[C];
         line_pairs<K, PART>(B.wave, i0, [&](int i, unsigned at, int) {
           if (MODE == PO_SCREEN) a[i] = pa[at];
@@ -264,7 +268,7 @@ k_plane_in(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__
       wave_fence();
       constexpr int G = PairGroup<K>::value;
 #pragma unroll 1
-      for (int i0 = 0; i0 < RP::CNT; i0 += G) {
+      for (int i0 = 0; i0 < PairGroup<K>::count(B.wave); i0 += G) {
         float2 q0[G], q1[G], q2[G], q3[G];
         line_pairs<K, PART>(B.wave, i0, [&](int i, unsigned at, int) {
           q0[i] = R[at];
