@@ -25,6 +25,18 @@ struct PL1 : PL<N1, N2> {
   static constexpr bool IO = PL<N1, N2>::W <= 4 || PL<N1, N2>::W == 8 || PL<N1, N2>::CH == 2;
 };
 
+// Whether a launch of this many blocks fills the chip well enough to beat the separate passes.  Up to four
+// waves a plane several blocks share a CU and it always does.  From five on a CU runs one block at a time, so
+// a launch takes whole rounds of 256 blocks: a last round that leaves the launch under two thirds full loses
+// (96 planes of three lanes are 288 blocks in two rounds: 96 x 256 x 192 920 -> 857 us a CG iteration without
+// the fused passes there, 96 x 128 x 256 626 -> 586), and so do fewer than 96 blocks of eight or ten waves
+// (the one-lane coefficient pass at 64 x 256 x 256: 12 us over the separate passes).
+template <class K>
+static bool fills(int blocks) {
+  const int rounds = (blocks + 255) / 256;
+  return K::W <= 4 || ((K::W * K::CH < 8 || blocks >= 96) && (rounds == 1 || 3 * blocks >= 2 * 256 * rounds));
+}
+
 // block, plane and lane of the three kernels: CH planes a block, in order
 template <class K>
 struct PlaneOf {
@@ -314,10 +326,27 @@ k_plane_in(const MemberDev* __restrict__ mem, Dims d, const float2* __restrict__
 // ---------------------------------------------------------------------------------------------
 int plane_blocks(const Dims& d) { return d.n0; }  // of the one-way kernels
 template <int N1, int N2>
-struct PlaneIo {
-  static int run() { return PL1<N1, N2>::IO ? 1 : 0; }
+struct PlaneCoefFills {
+  static int run(const LaunchCtx& c) { return fills<PL<N1, N2>>(c.nm * c.d.n0 / PL<N1, N2>::CH) ? 1 : 0; }
 };
-bool plane_io_supported(const Dims& d) { return dispatch_plane<PlaneIo>(d) == 1; }
+bool plane_coef_fills(const LaunchCtx& c) { return dispatch_plane<PlaneCoefFills>(c.d, c) == 1; }
+
+template <int N1, int N2>
+struct PlaneIoFills {
+  // cgupd: the x and r update reads four fields and writes two, so little is left to gain but the launch;
+  // one full round takes it, or two (192 x 256 x 192, three rounds: 49 us an iteration over the separate
+  // passes; 160 x 96 x 160, 480 blocks: 13 us under them)
+  static int run(const LaunchCtx& c, bool cgupd) {
+    using K = PL1<N1, N2>;
+    const int blocks = c.nm * c.d.n0;
+    const bool few = blocks <= 256 || (blocks >= 448 && blocks <= 512);
+    return K::IO && fills<K>(blocks) && (!cgupd || K::W <= 4 || few) ? 1 : 0;
+  }
+};
+bool plane_out_fills(const LaunchCtx& c) { return dispatch_plane<PlaneIoFills>(c.d, c, false) == 1; }
+bool plane_in_fills(const LaunchCtx& c, int mode) {
+  return dispatch_plane<PlaneIoFills>(c.d, c, mode == ZUM_CGUPD) == 1;
+}
 
 template <int N1, int N2>
 struct RunPlaneCoef {

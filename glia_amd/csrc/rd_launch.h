@@ -62,9 +62,12 @@ enum { ZUM_AXPBY = 0, ZUM_CGUPD = 1 };
 int launch_z_upd_r2c(const LaunchCtx& c, int mode, int ra, int rb, int rc, int rd, const double* sc, int s_out,
                      bool honor_done);
 // the elasticity passes fused over x-planes (plane_point.hip), on grids plane_supported takes:
-// F_yz(m F_yz^-1 in); where plane_io_supported, ZPM_SCREEN and ZPM_C2R_DOT with their Y pass
-// (plane_blocks(d) blocks of partials) and the two launch_z_upd_r2c modes with theirs
-bool plane_io_supported(const Dims& d);
+// F_yz(m F_yz^-1 in), ZPM_SCREEN and ZPM_C2R_DOT with their Y pass (plane_blocks(d) blocks of partials) and
+// the two launch_z_upd_r2c modes with theirs.  The *_fills say where they are faster than the separate passes
+// with c's lanes.
+bool plane_coef_fills(const LaunchCtx& c);
+bool plane_out_fills(const LaunchCtx& c);
+bool plane_in_fills(const LaunchCtx& c, int mode);
 int plane_blocks(const Dims& d);
 int launch_plane_coef(const LaunchCtx& c, int s_in, int s_out, int r_slot, bool honor_done);
 int launch_plane_out(const LaunchCtx& c, int mode, int s_in, int r_out, int r_b, bool honor_done);

@@ -131,7 +131,6 @@ int RDEnsemble::init() {
     }
   }
   plane_ = plane_supported(d_);
-  plane_io_ = plane_ && plane_io_supported(d_);
   if (!supported_line(d_.n0) || !supported_line(d_.n1) || !supported_z(d_.n2))
     return fail(-4, "unsupported grid: n0, n1 in {32,48,64,80,96,128,160,192,256}, n2 in {32,64,96,128,160,192,256}");
   if (z_blocks(d_) <= 0 || ((int64_t)d_.n0 * d_.n1) % z_lines_per_block(d_.m2) != 0)
@@ -705,7 +704,7 @@ int RDEnsemble::lin_coef_transform(const int* nterms, const int (*lane)[4], cons
   LaunchCtx c = ctx();
   const bool hd = honor_lanes_;
   GLIA_TRYC(launch_col_lin(c, nterms, lane, slot, dir, CS_T7, hd));
-  if (plane_) {
+  if (plane_ && plane_coef_fills(c)) {
     GLIA_TRYC(launch_plane_coef(c, CS_T7, CS_T7, coef_rs, hd));
   } else {
     GLIA_TRYC(launch_col_plain(c, 1, +1, CS_T7, CS_T7, hd));
@@ -721,7 +720,7 @@ int RDEnsemble::lin_screen_transform(const int* nterms, const int (*lane)[4], co
   LaunchCtx c = ctx();
   const bool hd = honor_lanes_;
   GLIA_TRYC(launch_col_lin(c, nterms, lane, slot, dir, CS_T7, hd));
-  if (plane_io_) {
+  if (plane_ && plane_out_fills(c)) {
     GLIA_TRYC(launch_plane_out(c, ZPM_SCREEN, CS_T7, out_rs, u_rs, hd));
   } else {
     GLIA_TRYC(launch_col_plain(c, 1, +1, CS_T7, CS_T7, hd));
@@ -734,7 +733,7 @@ int RDEnsemble::c2r_dots(int cs_in, int out_rs, int r_rs) {
   LaunchCtx c = ctx();
   const bool hd = honor_lanes_;
   GLIA_TRYC(launch_col_plain(c, 0, +1, cs_in, CS_T7, hd));
-  if (plane_io_) {
+  if (plane_ && plane_out_fills(c)) {
     GLIA_TRYC(launch_plane_out(c, ZPM_C2R_DOT, CS_T7, out_rs, r_rs, hd));
   } else {
     GLIA_TRYC(launch_col_plain(c, 1, +1, CS_T7, CS_T7, hd));
@@ -744,14 +743,14 @@ int RDEnsemble::c2r_dots(int cs_in, int out_rs, int r_rs) {
 }
 
 int RDEnsemble::lane_part_sum(int nq, double* out) {
-  GLIA_TRYC(launch_lane_part_sum(ctx(), plane_io_ ? plane_blocks(d_) : z_blocks(d_), nq, out));
+  GLIA_TRYC(launch_lane_part_sum(ctx(), plane_ && plane_out_fills(ctx()) ? plane_blocks(d_) : z_blocks(d_), nq, out));
   return 0;
 }
 
 int RDEnsemble::fft_r2c_axpby(int p_rs, int z_rs, int cs_out) {
   LaunchCtx c = ctx();
   const bool hd = honor_lanes_;
-  if (plane_io_) {
+  if (plane_ && plane_in_fills(c, ZUM_AXPBY)) {
     GLIA_TRYC(launch_plane_in(c, ZUM_AXPBY, p_rs, z_rs, -1, -1, nullptr, cs_out, hd));
   } else {
     GLIA_TRYC(launch_z_upd_r2c(c, ZUM_AXPBY, p_rs, z_rs, -1, -1, nullptr, cs_out, hd));
@@ -765,7 +764,7 @@ int RDEnsemble::fft_r2c_cgupd(int x_rs, int r_rs, int p_rs, int w_rs, const doub
   if (!sc) return fail(-2, "fft_r2c_cgupd needs the device scalar <p, A p>");
   LaunchCtx c = ctx();
   const bool hd = honor_lanes_;
-  if (plane_io_) {
+  if (plane_ && plane_in_fills(c, ZUM_CGUPD)) {
     GLIA_TRYC(launch_plane_in(c, ZUM_CGUPD, x_rs, r_rs, p_rs, w_rs, sc, cs_out, hd));
   } else {
     GLIA_TRYC(launch_z_upd_r2c(c, ZUM_CGUPD, x_rs, r_rs, p_rs, w_rs, sc, cs_out, hd));

@@ -323,9 +323,7 @@ class RDEnsemble {
     int kind;
     hipEvent_t a, b;
   };
-  // Y and Z passes fused over x-planes: of the matvec and the strain channels; of the elasticity CG's
-  // one-way transforms
-  bool plane_ = false, plane_io_ = false;
+  bool plane_ = false;  // Y and Z passes fused over x-planes
   int yf_split_ = 0, xf_split_ = 0;  // variants of the forward divergence passes (autotune)
   static constexpr int kYfVariants = 4;
   static constexpr int kXfVariants = 3;

@@ -131,10 +131,12 @@ def elastic(mu, lam, scr, avg):
 
 
 @pytest.mark.parametrize("n", [(32, 32, 32), (32, 48, 64), (32, 80, 160), (32, 96, 96), (32, 128, 128), (32, 160, 160),
-                               (32, 192, 160), (32, 256, 256)])
+                               (32, 192, 160), (32, 256, 256),
+                               (64, 160, 96), (96, 160, 96), (96, 96, 192)])
 def test_elasticity_on_planes(n):
     """Operator, preconditioner and a solve whose residual is measured with the FP64 operator; sizes with
-    whole and split planes, lines that do not fill a wave, and one whose one-way transforms stay separate."""
+    whole and split planes, lines that do not fill a wave, one whose one-way transforms stay separate, and the
+    mixes of fused and separate passes that launches of one and of three lanes take by how they fill the chip."""
     from glia_amd import elasticity
     from glia_amd.synth import tissue_and_tumor
     print("case plane elasticity", n, flush=True)
