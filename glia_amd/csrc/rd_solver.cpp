@@ -236,6 +236,7 @@ int RDEnsemble::alloc_member(int m) {
   GLIA_HIP(hipMalloc(&part_[m], sizeof(double) * nb));
   M.part = part_[m];
   GLIA_HIP(hipMalloc(&M.kmask, sizeof(unsigned) * (d_.n0 + 8)));
+  GLIA_HIP(hipMemsetAsync(M.kmask, 0xff, sizeof(unsigned) * (d_.n0 + 8), stream_));
   M.planes = M.kmask + d_.n0;
   int rc = alloc_history(m);
   if (rc) return rc;
@@ -1628,7 +1629,7 @@ int RDEnsemble::adjoint_end() {
 // holding both fields (0) or one group per field (1).  Y pass: one group holding three fields (0),
 // one group per field (1), or the fields split over blocks at 3 (2) or 2 (3) waves per SIMD.  The
 // choice is kept in a text cache (one line per device, grid and member count: "<arch> n0 n1 n2 nm
-// xf yf xf_ms0 xf_ms1 yf_ms0 yf_ms1 yf_ms2 yf_ms3") that later handles read instead of timing again.
+// xf yf xf_ms0 xf_ms1 xf_ms2 yf_ms0 yf_ms1 yf_ms2 yf_ms3") that later handles read instead of timing again.
 int RDEnsemble::autotune(const char* cache_path, int* choice) {
   hipDeviceProp_t prop;
   int dev = 0;
@@ -1654,6 +1655,8 @@ int RDEnsemble::autotune(const char* cache_path, int* choice) {
       }
     }
   }
+  // with the plane pass on the matvec's path there is nothing to choose: the defaults stand, with no times
+  if (plane_) return autotune_keep(cache_path, key.str(), nullptr, nullptr, choice);
   int rc = clear_done();  // every member's kernels run during the timing
   if (rc) return rc;
   hipEvent_t a, b;
@@ -1692,12 +1695,18 @@ int RDEnsemble::autotune(const char* cache_path, int* choice) {
   if (rc) return rc;
   xf_split_ = (int)(std::min_element(xf_ms, xf_ms + kXfVariants) - xf_ms);
   yf_split_ = (int)(std::min_element(yf_ms, yf_ms + kYfVariants) - yf_ms);
+  return autotune_keep(cache_path, key.str(), xf_ms, yf_ms, choice);
+}
+
+// the variants in force, returned and appended to the cache under key with their times (0: not timed)
+int RDEnsemble::autotune_keep(const char* cache_path, const std::string& key, const double* xf_ms, const double* yf_ms,
+                              int* choice) {
   if (choice) { choice[0] = xf_split_; choice[1] = yf_split_; }
   if (cache_path) {
     std::ofstream out(cache_path, std::ios::app);
-    out << key.str() << ' ' << xf_split_ << ' ' << yf_split_;
-    for (int v = 0; v < kXfVariants; v++) out << ' ' << xf_ms[v];
-    for (int v = 0; v < kYfVariants; v++) out << ' ' << yf_ms[v];
+    out << key << ' ' << xf_split_ << ' ' << yf_split_;
+    for (int v = 0; v < kXfVariants; v++) out << ' ' << (xf_ms ? xf_ms[v] : 0.0);
+    for (int v = 0; v < kYfVariants; v++) out << ' ' << (yf_ms ? yf_ms[v] : 0.0);
     out << '\n';
   }
   return 0;

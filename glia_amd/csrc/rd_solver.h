@@ -160,6 +160,7 @@ class RDEnsemble {
   // time the forward divergence variants on this handle (or read them from the cache file) and
   // keep the faster; choice (2 ints, may be NULL) receives (xf_split, yf_split)
   int autotune(const char* cache_path, int* choice);
+  int autotune_keep(const char* cache_path, const std::string& key, const double* xf_ms, const double* yf_ms, int* choice);
   void variants(int* xf, int* yf) const { *xf = xf_split_; *yf = yf_split_; }
   int smooth_field(int m, int rslot, double sigma);  // weierstrassSmoother, in place
   // the same smoother on any device field f of the grid, in place, through tmp (a distinct field

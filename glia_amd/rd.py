@@ -320,7 +320,8 @@ class RDSolver:
 
     def autotune(self, cache_path=None):
         """Time the variants of the forward divergence passes on this handle and keep the faster
-        (cache_path: a text file of earlier choices, read first and appended to).  Returns
+        (cache_path: a text file of earlier choices, read first and appended to).  Grids with n1 and n2
+        within a factor of two do not run these variants; nothing is timed there.  Returns
         (x_pass_split, y_pass_split)."""
         ch = (ctypes.c_int * 2)()
         path = None if cache_path is None else str(cache_path).encode()

@@ -311,7 +311,8 @@ int glia_rd_use_graphs(glia_rd_t h, int enable);
    file of earlier choices, read first and appended to.  choice (2 ints, may be NULL) receives
    (X-pass variant, Y-pass variant).  Call before the first solve; the results do not change
    beyond FP32 rounding.  On grids with n1 and n2 within a factor of two the diffusion operator runs
-   its Y and Z passes fused and these variants are not on its path. */
+   its Y and Z passes fused and these variants are not on its path: nothing is timed, the untuned
+   handle's variants are returned, and the file's line holds zeros for the times. */
 int glia_rd_autotune(glia_rd_t h, const char* cache_path, int* choice);
 /* Time steps replayed from captured graphs (glia_rd_use_graphs on, store-all history): each
    forward and adjoint step runs as one graph whose CG loops are unrolled to the counts of the

@@ -1,8 +1,9 @@
 """GPU parity on the headline grids: the 128- and 256-point line plans that the 128^3 and 256^3
 workloads run, against the FP64 oracle (through the C ABI).
 
-Every 256-point kernel is reached on grids with one long axis: 256 x 32 x 32 runs the X passes
-(k_xi_grad<256>, k_xf_div<256>), 32 x 256 x 32 the Y passes (k_yi_grad<256>, k_yf_div<256>) and
+Every 256-point kernel is reached on grids with one long axis: 256 x 32 x 32 runs the X passes around the
+plane pass (k_xi_grad<256>, the summing k_xf_div<256>), 256 x 32 x 96 those around the separate passes
+(k_xf_div<256> and its variants), 32 x 256 x 32 the Y passes (k_yi_grad<256>, k_yf_div<256>) and
 32 x 32 x 256 the Z passes on 128-point packed lines (k_z_diff<128>, k_z_point<128>,
 k_z_gradq<128>); the 128 analogues do the same for the 128-point plans.  The oracle finishes
 those in seconds.  The full 256^3 and 128^3 grids are checked against fixtures the oracle wrote
@@ -171,12 +172,18 @@ def test_headline_grid_gradient_vs_oracle_fixture(rd, name):
         assert abs(g[0][k] - go[k]) / max(abs(go[k]), 1e-2 * np.linalg.norm(go)) < 1e-4
 
 
-@pytest.mark.parametrize("split", ["none", "xf", "xf3", "yf", "yfb", "yfb2"])
-@pytest.mark.parametrize("n", [(32, 256, 32), (256, 32, 32), (32, 128, 32)])
+SPLITS = ["none", "xf", "xf3", "yf", "yfb", "yfb2"]
+# the X variants run where n1 and n2 are more than a factor of two apart; 256 x 32 x 32 takes the plane pass
+# under every setting
+VARIANT_GRIDS = [(n, split) for n in [(32, 256, 32), (256, 32, 32), (32, 128, 32)] for split in SPLITS] + \
+    [(n, split) for n in [(48, 32, 96), (128, 32, 96), (160, 32, 96), (256, 32, 96)] for split in ("none", "xf", "xf3")]
+
+
+@pytest.mark.parametrize("n,split", VARIANT_GRIDS)
 def test_divergence_variants_headline_plans_vs_oracle(rd, oracle_mod, n, split):
     """Every variant of the forward divergence passes the autotuner may choose (GLIA_SPLIT_DIV) on
-    the long-axis grids that run it at 128 or 256 points: applyD within 1e-5 and J, dJ within the
-    oracle bars (nt = 2)."""
+    grids that run the Y variants at 128 or 256 points and the X variants at 48 to 256: applyD within 1e-5 and
+    J, dJ within the oracle bars (nt = 2), and the passes meant are the ones that ran."""
     import os
     print("case variant", n, split, flush=True)
     dt, nt = 0.02, 2
@@ -207,7 +214,13 @@ def test_divergence_variants_headline_plans_vs_oracle(rd, oracle_mod, n, split):
     ed = rel(s.get_field(0, "ct"), ref_d)
     s.set_data(0, d1, None, -0.99)
     J, g = s.objective_and_gradient([x])
+    s.profile(True)
+    s.solve_state(0)
+    prof = s.profile_get()
+    s.profile(False)
     s.close()
+    separate = max(n[1], n[2]) > 2 * min(n[1], n[2])
+    assert (prof["xf_matvec"][0] > 0) == separate and (prof["plane_div"][0] > 0) != separate
     print("applyD %.2e J %.2e dJ %.2e" % (ed, abs(J[0] - Jo) / abs(Jo), rel(g[0], go)), flush=True)
     assert ed < 1e-5
     assert abs(J[0] - Jo) / abs(Jo) < 1e-5

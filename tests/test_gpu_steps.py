@@ -141,6 +141,90 @@ def test_autotune_choice_cache_and_results(members, tmp_path, oracle_mod):
     assert rel(gt[0], go) < 1e-4
 
 
+def test_autotune_times_nothing_where_the_variants_are_not_on_the_path(tmp_path):
+    """Grids whose matvec takes the plane pass: the untuned variants, a cache line without times, and no solver
+    kernel timed."""
+    from glia_amd import rd
+    n = (96, 64, 64)
+    print("case autotune plane", n, flush=True)
+    cache = tmp_path / "tune.txt"
+    s = rd.RDSolver(n)
+    assert s.autotune(str(cache)) == (0, 0)
+    s.close()
+    line = open(cache).read().split()
+    assert len(line) == 14 and all(float(t) == 0.0 for t in line[7:])
+    s = rd.RDSolver(n)
+    assert s.autotune(str(cache)) == (0, 0) and len(open(cache).read().splitlines()) == 1
+    s.close()
+
+
+@pytest.mark.parametrize("n", [(64, 32, 96), (96, 32, 96)])
+def test_autotune_and_variants_on_separate_passes(tmp_path, oracle_mod, n):
+    """Grids whose matvec runs the separate passes (n1 and n2 more than a factor of two apart): the choice is the
+    fastest of the times in the cache, and every variant gives the oracle's J and dJ."""
+    from glia_amd import rd, synth
+    print("case autotune separate", n, flush=True)
+    pr = synth.problem(n, 41, nbases=6, nnz=4, kappa=0.03, rho=7.0)
+    pr["d1"] = (pr["wm"] > 0.6).astype(np.float32)
+    x = [np.concatenate([pr["p"], [pr["kappa"], pr["rho"]]])]
+
+    def handle(split=None):
+        old = os.environ.pop("GLIA_SPLIT_DIV", None)
+        if split:
+            os.environ["GLIA_SPLIT_DIV"] = split
+        try:
+            s = rd.RDSolver(n, dt=DT, nt=2, k_gm_wm=0.2, r_gm_wm=0.2, beta=1e-3)
+        finally:
+            os.environ.pop("GLIA_SPLIT_DIV", None)
+            if old is not None:
+                os.environ["GLIA_SPLIT_DIV"] = old
+        s.set_tissue(0, pr["wm"], pr["gm"], pr["csf"], pr["vt"])
+        s.set_coefficients(0, pr["kappa"], pr["rho"])
+        s.set_basis(0, pr["centers"], pr["sigma"])
+        s.set_data(0, pr["d1"], None, -0.99)
+        return s
+
+    o = oracle_mod.Oracle(n)
+    o.set_tissue(pr["wm"], pr["gm"], pr["csf"], pr["vt"])
+    o.set_time(DT, 2)
+    o.set_k(pr["kappa"], 0.2, 0.0)
+    o.set_rho(pr["rho"], 0.2, 0.0)
+    o.prec_factor()
+    o.set_phi(pr["centers"], pr["sigma"], 1.0, False)
+    o.set_data(pr["d1"].astype(np.float64), None, -0.99)
+    o.set_opt(beta=1e-3)
+    o.set_time(DT, 2)
+    Jo, go = o.objective_and_gradient(x[0], mode=2)
+
+    cache = tmp_path / "tune.txt"
+    s = handle()
+    choice = s.autotune(str(cache))
+    line = open(cache).read().split()
+    ms = [float(t) for t in line[7:]]
+    assert len(ms) == 7 and min(ms) > 0.0
+    assert choice == (int(np.argmin(ms[:3])), int(np.argmin(ms[3:]))) and line[5:7] == [str(c) for c in choice]
+    s.close()
+    s = handle()
+    assert s.autotune(str(cache)) == choice and len(open(cache).read().splitlines()) == 1
+    s.close()
+    by_split = {}
+    for split in ("none", "xf", "xf3", "yf", "both", "yfb", "xf,yfb2"):
+        s = handle(split)
+        J, g = s.objective_and_gradient(x)
+        s.profile(True)
+        s.objective_and_gradient(x)
+        prof = s.profile_get()
+        s.profile(False)
+        s.close()
+        assert prof["xf_matvec"][0] > 0 and prof["yf_div"][0] > 0 and prof["xf_sum"][0] == 0, split
+        assert abs(J[0] - Jo) / abs(Jo) < 1e-5, split
+        assert rel(g[0], go) < 1e-4, split
+        by_split[split] = (J[0], g[0])
+    # the X pass in three groups takes the operations of the two-group pass: the same bits
+    assert by_split["xf3"][0] == by_split["xf"][0]
+    assert np.array_equal(by_split["xf3"][1], by_split["xf"][1])
+
+
 def test_lockstep_group_equals_separate_bitwise():
     """Handles of different grids, member counts, nt and history modes evaluated in lockstep
     (glia_rd_objective_and_gradient_lockstep: time step i of every handle in one graph) give J and
