@@ -269,10 +269,21 @@ struct RealPart {
   static constexpr int PM = K::M / PARTS;        // pairs per line and part
   static constexpr int CNT = 32 * PM / 64;       // pairs per lane and part
 };
+// The lane number for a part's addresses.  On 256 lines of 160 reals the quotients by a part's 20 pairs a
+// line, kept from one part to the next beside 64 values a lane, spilled 170 registers: it is renewed there and
+// they are made again, 77 spills (CN solves of 4 x 160 x 256 x 160 with a scan's zeros 9.85 -> 9.32 ms, with a
+// coefficient zero nowhere 6.46 -> 6.03).  With fewer values a lane it costs 2%, at 24 pairs a line it is even.
+template <class K>
+__device__ __forceinline__ int part_lane() {
+  using RP = RealPart<K>;
+  int lane = (int)threadIdx.x & 63;
+  if constexpr (RP::PARTS > 1 && RP::PM % 8 != 0 && K::RY == 64) asm volatile("" : "+v"(lane));
+  return lane;
+}
 template <class K, int PART, int HP>
 __device__ __forceinline__ void real_fetch(float2 (&q)[RealPart<K>::CNT], GPtrT<HP> field, const PlaneLane& L) {
   using RP = RealPart<K>;
-  const int lane = (int)threadIdx.x & 63;
+  const int lane = part_lane<K>();
   const int wave = __builtin_amdgcn_readfirstlane(L.zl >> 5);
   const auto f0 = field + (wave * 32 * K::M + PART * RP::PM);
 #pragma unroll
@@ -290,7 +301,7 @@ __device__ __forceinline__ void real_fetch(float2 (&q)[RealPart<K>::CNT], GPtrT<
 template <class K, int PART, class Fn>
 __device__ __forceinline__ void real_use(float* lds, const float2 (&q)[RealPart<K>::CNT], const PlaneLane& L, Fn fn) {
   using RP = RealPart<K>;
-  const int lane = (int)threadIdx.x & 63;
+  const int lane = part_lane<K>();
   const int l0 = L.zl & ~31;
   wave_fence();  // the wave's earlier reads of its rows come first
 #pragma unroll
