@@ -20,9 +20,11 @@ template <int N1, int N2>
 struct PL1 : PL<N1, N2> {
   static constexpr int CH = 1, TB = PL<N1, N2>::T;
   static constexpr int MINW = 2;
-  // worth it where more than one block runs on a CU or eight waves fill it: at 192 points (six waves, one
-  // block a CU) the separate passes are the faster ones, a 192^3 solve 79.7 against 81.6 ms
-  static constexpr bool IO = PL<N1, N2>::W <= 4 || PL<N1, N2>::W == 8 || PL<N1, N2>::CH == 2;
+  // Where more waves hold the lines than the columns at 40 entries a lane, 192 x 160 and 256 x 160, the separate
+  // passes are the faster ones as soon as a launch takes a second round (128 x 192 x 160, a CG iteration 666
+  // against 691 us, 192 x 192 x 160 934 against 1015; 80 x 256 x 160, one round, 605 against 570).
+  using Q = PL<N1, N2>;
+  static constexpr bool ONE_ROUND = Q::WZ > Q::WY && Q::RZ == 40;
 };
 
 // Whether a launch of this many blocks fills the chip well enough to beat the separate passes.  Up to four
@@ -340,7 +342,8 @@ struct PlaneIoFills {
     using K = PL1<N1, N2>;
     const int blocks = c.nm * c.d.n0;
     const bool few = blocks <= 256 || (blocks >= 448 && blocks <= 512);
-    return K::IO && fills<K>(blocks) && (!cgupd || K::W <= 4 || few) ? 1 : 0;
+    if (K::ONE_ROUND && blocks > 256) return 0;
+    return fills<K>(blocks) && (!cgupd || K::W <= 4 || few) ? 1 : 0;
   }
 };
 bool plane_out_fills(const LaunchCtx& c) { return dispatch_plane<PlaneIoFills>(c.d, c, false) == 1; }
