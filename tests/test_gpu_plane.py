@@ -1,7 +1,7 @@
-"""The plane pass of the diffusion operator against an FP64 FFT on the CPU: every square size and
-rectangular ones (lines that do not fill a wave, more waves in one layout than in the other, two planes
-a block), with a coefficient that vanishes on whole planes, on whole groups of 32 lines and on
-parts of a group, and one that vanishes nowhere."""
+"""The plane pass of the diffusion operator against an FP64 FFT on the CPU: every pair of sides (lines that
+do not fill a wave, more waves in one layout than in the other, two planes a block) and the pairs next to the
+rule's border, with a coefficient that vanishes on whole planes, on whole groups of 32 lines and on
+parts of a group, and one that vanishes nowhere; every X length with planes left out."""
 import numpy as np
 import pytest
 
@@ -33,10 +33,13 @@ def fields(n, kind, rng):
     return k.astype(np.float32)
 
 
+# every pair of sides that has a plane pass (within a factor of two)
+SIDES = [(a, b) for a in (32, 48, 64, 80, 96, 128, 160, 192, 256) for b in (32, 64, 96, 128, 160, 192, 256)
+         if max(a, b) <= 2 * min(a, b)]
+
+
 @pytest.mark.parametrize("kind", ["dense", "sparse"])
-@pytest.mark.parametrize("n", [(32, 32, 32), (48, 64, 64), (32, 96, 96), (80, 128, 128), (32, 160, 160), (32, 192, 192),
-                               (32, 256, 256), (32, 48, 64), (48, 80, 160), (32, 96, 64), (32, 96, 192),
-                               (32, 128, 256), (32, 160, 128), (32, 192, 96), (32, 256, 192)])
+@pytest.mark.parametrize("n", [(32, a, b) for a, b in SIDES] + [(48, 64, 64), (80, 128, 128), (48, 80, 160)])
 def test_operator_on_planes(n, kind):
     from glia_amd import rd
     print("case plane", n, kind, flush=True)
@@ -85,6 +88,35 @@ def test_operator_with_planes_left_out(n, kind):
     s.close()
 
 
+@pytest.mark.parametrize("kind", ["dense", "sparse"])
+@pytest.mark.parametrize("n,plane", [((32, 32, 64), True), ((32, 32, 96), False), ((32, 64, 32), True), ((32, 80, 32), False),
+                                     ((32, 128, 64), True), ((32, 160, 64), False), ((32, 48, 96), True),
+                                     ((32, 48, 128), False), ((32, 128, 256), True), ((32, 96, 256), False)])
+def test_operator_at_the_rules_border(n, plane, kind):
+    """Sides within a factor of two take the plane pass, the next ones the separate passes: the same operator."""
+    from glia_amd import rd
+    print("case plane border", n, kind, flush=True)
+    rng = np.random.default_rng([n[1], n[2], len(kind)])
+    s = rd.RDSolver(n)
+    s.set_coefficients(0, 0.05, 8.0)
+    s.precFactor()
+    f = rng.standard_normal(n).astype(np.float32)
+    s.set_field(0, "work", f)
+    s.profile(True)
+    s.diffusion_solve("work", 0.01)
+    prof = s.profile_get()
+    s.profile(False)
+    assert (prof["plane_div"][0] > 0) == plane and (prof["z_diff"][0] > 0) != plane
+    k = fields(n, kind, rng)
+    s.set_field(0, "k", k)
+    s.set_field(0, "work", f)
+    s.apply_d("work", "ct")
+    ref = apply_d(k.astype(np.float64), f.astype(np.float64))
+    err = np.linalg.norm(s.get_field(0, "ct") - ref) / np.linalg.norm(ref)
+    assert err < 5e-6, err  # the bound of test_operator_on_planes
+    s.close()
+
+
 def test_zero_coefficient_and_a_field_written_after_creation():
     """All planes skipped gives exactly zero, and the skip follows a coefficient changed in place."""
     from glia_amd import rd
@@ -130,13 +162,11 @@ def elastic(mu, lam, scr, avg):
     return A, B
 
 
-@pytest.mark.parametrize("n", [(32, 32, 32), (32, 48, 64), (32, 80, 160), (32, 96, 96), (32, 128, 128), (32, 160, 160),
-                               (32, 192, 160), (32, 256, 256),
-                               (64, 160, 96), (96, 160, 96), (96, 96, 192)])
+@pytest.mark.parametrize("n", [(32, a, b) for a, b in SIDES] + [(64, 160, 96), (96, 160, 96), (96, 96, 192)])
 def test_elasticity_on_planes(n):
-    """Operator, preconditioner and a solve whose residual is measured with the FP64 operator; sizes with
-    whole and split planes, lines that do not fill a wave, one whose one-way transforms stay separate, and the
-    mixes of fused and separate passes that launches of one and of three lanes take by how they fill the chip."""
+    """Operator, preconditioner and a solve whose residual is measured with the FP64 operator; every
+    pair of sides, and the mixes of fused and separate passes that launches of one and of three lanes take by how
+    they fill the chip."""
     from glia_amd import elasticity
     from glia_amd.synth import tissue_and_tumor
     print("case plane elasticity", n, flush=True)

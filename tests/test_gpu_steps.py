@@ -92,6 +92,37 @@ def test_captured_steps_equal_eager_steps_bitwise(members, adjoint_store):
             assert np.array_equal(a, b), name
 
 
+def test_captured_steps_of_a_large_grid_equal_eager_steps_bitwise():
+    """From 2^22 points times members a step without a budget of its own runs eagerly: the first evaluation
+    launches no captured step, later ones do, and each equals the eager handle's bit for bit, with x moved
+    between them."""
+    from glia_amd import rd, synth
+    print("case captured large", flush=True)
+    n, nt = 128, 3
+    prs = [synth.problem(n, seed, nbases=4, nnz=None) for seed in (5, 6)]
+    res = {}
+    for graphs in (False, True):
+        s = rd.RDSolver(n, nmembers=2, dt=DT, nt=nt, k_gm_wm=0.2, r_gm_wm=0.2)
+        for m, pr in enumerate(prs):
+            s.set_tissue(m, pr["wm"], pr["gm"], pr["csf"], pr["vt"])
+            s.set_coefficients(m, pr["kappa"], pr["rho"])
+            s.set_basis(m, pr["centers"], pr["sigma"])
+            s.set_data(m, (pr["wm"] > 0.5).astype(np.float32), None, -0.99)
+        s.use_graphs(graphs)
+        out, launched = [], []
+        for t in range(3):
+            out.append(s.objective_and_gradient([x * (1.0 + 0.1 * t) for x in xs(prs)]))
+            launched.append(s.step_info()[0])
+        print("graphs", graphs, "steps launched", launched, flush=True)
+        assert launched == [0, 2 * nt, 4 * nt] if graphs else launched == [0, 0, 0]
+        res[graphs] = out
+        s.close()
+    for (J0, g0), (J1, g1) in zip(res[False], res[True]):
+        assert np.array_equal(J0, J1)
+        for a, b in zip(g0, g1):
+            assert np.array_equal(a, b)
+
+
 def test_autotune_choice_cache_and_results(members, tmp_path, oracle_mod):
     """The autotuner picks a variant per forward divergence pass, writes it to the cache, and a
     later handle reads the cache instead of timing again; every variant combination evaluates to
