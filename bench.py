@@ -876,16 +876,24 @@ def main():
     prof = s.profile_get()
     s.profile(False)
     its_p = sum(s.stats(m)["pcg_iterations"] for m in range(M))
+    solves_p = sum(s.stats(m)["cn_solves"] for m in range(M))
     field_bytes = 4.0 * n ** 3
+    # the share of the x-planes that the matvec's passes read and write (the others hold no nonzero k)
+    on_planes = prof["plane_div"][0] > 0 and M * n ** 3 >= 1 << 21
+    active = float(np.mean([(s.get_field(m, "k") != 0).any(axis=(1, 2)).mean() for m in range(M)])) if on_planes else 1.0
     dom = max(prof, key=lambda k: prof[k][1])
     cnt, ms = prof[dom]
-    achieved = _lib.KERNEL_FIELDS[dom] * field_bytes * its_p / (ms / 1000.0) / 1e9
+    achieved = _lib.kernel_fields(dom, active) * field_bytes * its_p / (ms / 1000.0) / 1e9
     kernels = {k: {"launches": v[0], "ms": round(v[1], 3), "member_iterations": its_p,
-                   "GBs": round(_lib.KERNEL_FIELDS[k] * field_bytes * its_p / (v[1] / 1000.0) / 1e9, 1)}
+                   "GBs": round(_lib.kernel_fields(k, active) * field_bytes * its_p / (v[1] / 1000.0) / 1e9, 1)}
                for k, v in prof.items() if v[0] > 0}
-    # whole-evaluation model of algorithmic bytes: B = R [nt (230 + 144 m) + 20 (nt + 1)] per member
-    b_eval = field_bytes * (nt * (230 + 144 * mbar) + 20 * (nt + 1))
-    model_gbs = b_eval * M * args.steps / (t2 - t1) / 1e9
+    # algorithmic bytes of the CG solves of one evaluation (the passes of every iteration, and of each solve's
+    # first residual: no p update, no x and r update) over the whole evaluation's wall time
+    passes = [k for k, v in prof.items() if v[0] > 0]
+    f_it = sum(_lib.kernel_fields(k, active) for k in passes)
+    f_set = sum(_lib.kernel_fields(k, active) for k in passes if k != "pcg_update") - 2
+    b_eval = field_bytes * (its_p * f_it + solves_p * f_set)
+    model_gbs = b_eval * args.steps / (t2 - t1) / 1e9
     c0_member0 = s.get_field(0, "c0").astype(np.float64)
     k0, rho0, mask0 = s.get_field(0, "k"), s.get_field(0, "rho"), s.get_field(0, "filter")
     del s
@@ -987,8 +995,9 @@ def main():
                   "evaluation with HIP events around each CG kernel launch (graph replay off)",
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "algorithmic_bytes_per_launch": _lib.KERNEL_FIELDS[dom] * field_bytes * M,
+                     "algorithmic_bytes_per_launch": _lib.kernel_fields(dom, active) * field_bytes * M,
                      "traffic": traffic_from_profiles(dom, n, M)},
+        "active_planes": round(active, 4),
         "cpu_baseline": cpu,
         "plain_value": None if plain is None else round(plain, 4),
         "batched_vs_plain": None if plain is None else round(value / plain, 3),

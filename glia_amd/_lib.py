@@ -295,9 +295,18 @@ ME_SIGNATURES = {
 KERNELS = ["xi_pupd", "yi_grad", "z_diff", "yf_div", "xf_matvec", "pcg_update", "plane_div", "xf_sum"]
 # algorithmic bytes of one launch per member, in units of one field (4 n0 n1 n2 bytes): every
 # input read once and every output written once.  Grids with n1 and n2 within a factor of two run
-# plane_div and xf_sum in place of yi_grad, z_diff, yf_div and xf_matvec; plane_div does not read or transform planes where k is zero
+# plane_div and xf_sum in place of yi_grad, z_diff, yf_div and xf_matvec
 KERNEL_FIELDS = {"xi_pupd": 5, "yi_grad": 5, "z_diff": 7, "yf_div": 5, "xf_matvec": 4, "pcg_update": 6,
                  "plane_div": 6, "xf_sum": 5}
+# of these, the fields of which only the x-planes where k is not zero are read or written (grids with
+# plane_div, from 2^21 points times members)
+KERNEL_PLANE_FIELDS = {"xi_pupd": 2, "plane_div": 6, "xf_sum": 3}
+
+
+def kernel_fields(kernel, active=1.0):
+    """Fields one launch of a CG kernel moves per member; active is the share of the x-planes with a nonzero k
+    (1 where every plane is passed through memory)."""
+    return KERNEL_FIELDS[kernel] - KERNEL_PLANE_FIELDS.get(kernel, 0) * (1.0 - active)
 
 _lib = None
 
