@@ -667,7 +667,7 @@ def masseffect_config(args):
     steps and the loop stops); one step = one whole forward (nt + 1 = 41 time steps, 42 elasticity
     solves).
     Algorithmic bytes per time step, in fields of 4 N^3 bytes: 167 per elasticity CG iteration,
-    55 + 36 m per diffusion solve of m CG iterations, and 270 for the rest (elasticity set-up
+    45 + 22 m per diffusion solve of m CG iterations, and 270 for the rest (elasticity set-up
     with the initial residual 150: force 10, material 10, operator and preconditioner 130; CFL 3,
     coefficients 6, velocity staging 6, trajectories and div v 14, advection of five fields 14,
     copies back 10, transforms around the diffusion solve 4, reaction 3, velocity 12, its
@@ -693,7 +693,7 @@ def masseffect_config(args):
     steps = info["steps"]
     R = 4.0 * n ** 3
     m_diff = info["diff_iterations"] / max(steps, 1)
-    bytes_fwd = R * (167.0 * info["el_iterations"] + steps * (55.0 + 36.0 * m_diff + 270.0))
+    bytes_fwd = R * (167.0 * info["el_iterations"] + steps * (45.0 + 22.0 * m_diff + 270.0))
     achieved = bytes_fwd / t / 1e9
     line = {
         "metric": "mass-effect forward time steps/s at 160^3 (model 4)",
@@ -721,7 +721,7 @@ def multispecies_config(args):
     tumor seed and coefficients of the model-4 configuration, the reference's species parameters,
     forcing factor 6e4 and the model's CFL limit 8; one step = one whole forward (41 time steps).
     Algorithmic bytes per time step, in fields of 4 N^3 bytes: 167 per elasticity CG iteration,
-    55 + 36 m per diffusion solve of m CG iterations, and 330 for the rest (the 270 of the model-4
+    45 + 22 m per diffusion solve of m CG iterations, and 330 for the rest (the 270 of the model-4
     step, two more advected fields 6, k and its mean 10, clipping 14, the smoothing of i 8, D i 22)."""
     from glia_amd.mass_effect import MassEffectSolver
     from glia_amd.synth import mass_effect_case
@@ -744,7 +744,7 @@ def multispecies_config(args):
     steps = info["steps"]
     R = 4.0 * n ** 3
     m_diff = info["diff_iterations"] / max(steps, 1)
-    bytes_fwd = R * (167.0 * info["el_iterations"] + steps * (55.0 + 36.0 * m_diff + 330.0))
+    bytes_fwd = R * (167.0 * info["el_iterations"] + steps * (45.0 + 22.0 * m_diff + 330.0))
     achieved = bytes_fwd / t / 1e9
     line = {
         "metric": "multispecies mass-effect forward time steps/s at 160^3 (model 5)",
