@@ -233,11 +233,12 @@ int RDEnsemble::alloc_member(int m) {
   int64_t nb = std::max<int64_t>((int64_t)xf_div_blocks(d_) * 3, (int64_t)z_blocks(d_) * 2);
   nb = std::max<int64_t>(nb, (int64_t)pcg_update_blocks() * 2);
   nb = std::max<int64_t>(nb, (int64_t)ew_blocks() * 2);
-  GLIA_HIP(hipMalloc(&part_[m], sizeof(double) * nb));
+  const size_t mb = sizeof(unsigned) * (d_.n0 + 8);  // the planes' masks and bits, in the same allocation
+  GLIA_HIP(hipMalloc(&part_[m], sizeof(double) * nb + mb));
   M.part = part_[m];
-  GLIA_HIP(hipMalloc(&M.kmask, sizeof(unsigned) * (d_.n0 + 8)));
-  GLIA_HIP(hipMemsetAsync(M.kmask, 0xff, sizeof(unsigned) * (d_.n0 + 8), stream_));
+  M.kmask = reinterpret_cast<unsigned*>(part_[m] + nb);
   M.planes = M.kmask + d_.n0;
+  GLIA_HIP(hipMemsetAsync(M.kmask, 0xff, mb, stream_));
   int rc = alloc_history(m);
   if (rc) return rc;
   M.kr_gm = (float)cfg_.k_gm_wm;
@@ -416,7 +417,6 @@ RDEnsemble::~RDEnsemble() {
     free_history(m);
     (void)hipFree(st_[m]);
     (void)hipFree(part_[m]);
-    (void)hipFree(mh_[m].kmask);
     (void)hipFree(bricks_dev_[m]);
     (void)hipFree(brick_data_[m]);
     (void)hipFree(phi_scale_dev_[m]);
