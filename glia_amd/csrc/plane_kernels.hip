@@ -5,8 +5,11 @@
 // few to cover a block's loads and stores with arithmetic.  Measured against the three passes it
 // replaces, matvec middle of one CG iteration with every member active: 16 x 128^3 450 -> 193 us,
 // 8 x 160^3 424 -> 252, 8 x 192^3 726 -> 442, 8 x 256^3 1761 -> 882 (17 fields of traffic became 6).
-// Whole CN solves of four members on 96 x n1 x n2 grids: 1.05 to 1.35 times as fast at every size built
-// (96 x 96 1.38 -> 1.02 ms, 160 x 96 1.99 -> 1.74, 192 x 128 3.18 -> 2.83, 256 x 160 6.47 -> 6.17).
+// Whole CN solves of one and five members on 32, 96 and 256 x n1 x n2 grids, a scan's ellipsoid in the box: 1.16
+// times as fast in the mean, 0.99 (one member, 32 x 256 x 192) to 1.35 (5 x 256 x 128 x 128).  With a coefficient
+// that is zero nowhere 1.06 in the mean, 0.84 (5 x 256 x 160 x 96) to 1.23: pairs of sides where one layout leaves
+// waves idle lose there.  The sides alone decide: the host does not know k, and members of an ensemble with
+// different zeros must give the bits they give alone.
 #include "plane_fft.h"
 
 namespace glia {
