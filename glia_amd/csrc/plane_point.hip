@@ -5,9 +5,9 @@
 // Bound as the diffusion operator's plane pass: the vector units up to 128 points, the few waves a CU
 // holds beyond; and at 160^3 and below by the number of blocks, three planes for each of n0.  160^3, one
 // CG iteration: the three strain channels 197 -> 140 us, p's update and transform 59 -> 50, the screened
-// output 68 -> 65, the preconditioner's output 53 -> 51, x and r's update and transform 80 -> 81.  Whole
-// solves: 32^3 5.41 -> 4.32 ms, 64^3 7.13 -> 5.92, 96^3 16.2 -> 12.6, 128^3 23.8 -> 20.3, 160^3 50.9 ->
-// 46.6, 192^3 82.6 -> 79.7, 256^3 138 -> 130, 96 x 128 x 64 14.0 -> 12.0.
+// output 68 -> 65, the preconditioner's output 53 -> 51, x and r's update and transform 79 -> 87
+// (two rounds of blocks).  Whole solves: 32^3 5.41 -> 4.32 ms, 64^3 7.13 -> 5.92, 96^3 16.2 -> 12.6, 128^3 23.8 ->
+// 20.3, 160^3 50.9 -> 46.6, 192^3 82.6 -> 77.5, 256^3 138 -> 130, 96 x 128 x 64 14.0 -> 12.0.
 #include "plane_fft.h"
 
 #include <type_traits>
